@@ -1089,6 +1089,28 @@ hipError_t launch_gemm_i8(const GemmI8Args& a, int tile, hipStream_t s) {
   if (a.M <= 0 || a.N <= 0) return hipSuccess;
   if (a.epi == EPI_QSYNC) return launch_qsync(a, tile > 0 && tile <= kI8TileConfigs ? tile : 7, s);
   if (tile <= 0 || tile > kI8TileConfigs) {
+    if (const int small = pick_small_tile(a.M, a.N, 0)) {
+      GemmSmallArgs g{};
+      g.A = a.A;
+      g.lda = a.lda;
+      g.B = a.B;
+      g.ldb = a.ldb;
+      g.M = a.M;
+      g.N = a.N;
+      g.kbytes = a.K;
+      g.row_scales = a.row_scales;
+      g.col_scales = a.col_scales;
+      g.colsum = a.colsum;
+      g.bias = a.bias;
+      g.out = a.out;
+      g.out_lo = a.out_lo;
+      g.ldo = a.ldo;
+      g.act = a.act;
+      g.epi = a.epi;
+      g.row_absmax = a.row_absmax;
+      g.rs_out = a.rs_out;
+      return launch_gemm_small_i8(g, small, s);
+    }
     tile = pick_i8_tile(a.M, a.N, a.K, a.epi);
     if (tile == 13 && !a.Bf) tile = 9;  // no fragment-ordered image of B
   }

@@ -448,8 +448,29 @@ hipError_t launch_gemm_planes(const GemmPlArgs& a, int a_terms, int b_terms, int
                               hipStream_t s) {
   if (a.M <= 0 || a.N <= 0) return hipSuccess;
   if (a.lda % 64 != 0 || a.ldb % 64 != 0) return hipErrorInvalidValue;
-  if (tile <= 0 || tile > kPlanesTileConfigs)
+  if (tile <= 0 || tile > kPlanesTileConfigs) {
+    if (const int small = pick_small_tile(a.M, a.N, a_terms + b_terms)) {
+      GemmSmallArgs g{};
+      g.A = a.Ah;
+      g.Al = a.Al;
+      g.lda = 2 * a.lda;
+      g.B = a.Bh;
+      g.Bl = a.Bl;
+      g.ldb = 2 * a.ldb;
+      g.M = a.M;
+      g.N = a.N;
+      g.kbytes = 2 * a.K;
+      g.col_scales = a.col_scales;
+      g.bias = a.bias;
+      g.out = a.Ch ? static_cast<void*>(a.Ch) : static_cast<void*>(a.C);
+      g.out_lo = a.Cl;
+      g.ldo = a.ldc;
+      g.act = a.act;
+      g.epi = a.Ch ? EPI_PLANES : EPI_F32;
+      return launch_gemm_small_planes(g, a_terms, b_terms, small, s);
+    }
     tile = pick_planes_tile(a.M, a.N, a.K, a_terms, b_terms);
+  }
   if (a_terms == 1 && b_terms == 1) {
     switch (tile) {
       case 1: return launch_pl<256, 256, 4, 1, 1>(a, s);

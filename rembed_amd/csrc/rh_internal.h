@@ -210,6 +210,33 @@ struct GemmPlArgs {
   float qk_eps = 0.0f;
 };
 
+// The GEMMs of few rows (gemm_small.hip): u8 rows x s8 weights, or bf16 planes.
+struct GemmSmallArgs {
+  const void* A;    // u8 rows, or the hi plane
+  const void* Al;   // lo plane (two activation terms)
+  int lda;          // bytes
+  const void* B;    // s8 rows [Np][ldb], or the hi plane
+  const void* Bl;   // lo plane (fp32 weights)
+  int ldb;          // bytes
+  int M, N, kbytes; // kbytes: bytes of one row's K elements
+  const float* row_scales;  // int8: [M]
+  const float* col_scales;  // [N] or null (fp32)
+  const int32_t* colsum;    // EPI_ACC
+  const float* bias;        // [N] or null
+  void* out;        // per epi (I8Epi; EPI_F32 and EPI_PLANES for the planes)
+  void* out_lo;     // EPI_PLANES: lo plane or null
+  int ldo;          // elements
+  int act, epi;
+  float* row_absmax;  // as GemmI8Args
+  float* rs_out;
+};
+// 0 where the tiled kernels are ahead, else the tile of the few-row kernel.
+// terms: 0 for int8, else a_terms + b_terms of the planes product.
+int pick_small_tile(int M, int N, int terms);
+hipError_t launch_gemm_small_i8(const GemmSmallArgs& a, int tile, hipStream_t s);
+hipError_t launch_gemm_small_planes(const GemmSmallArgs& a, int a_terms, int b_terms, int tile,
+                                    hipStream_t s);
+
 // The split hi/lo of one value; every producer of activation planes uses
 // exactly this, so planes written by a producer equal launch_split_bf16's.
 __device__ __forceinline__ void split_hi_lo(float x, __bf16& hi, __bf16& lo) {

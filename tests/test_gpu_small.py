@@ -1,0 +1,155 @@
+"""The few-row GEMMs (gemm_small.hip) at the edges of their tiles and shares.
+
+M covers the 16-, 32- and 64-row tiles and their remainders, N the column tiles
+with a ragged last one (and grids that send a mode to its next tile or to the
+tiled kernels), K one element, less than one 64-byte step, steps that leave
+waves without a share, ragged ends and the deep linears.
+"""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from rembed_amd import _lib
+from rembed_amd import tensor as T
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1, 1, 16), (1, 768, 2304), (15, 30, 48), (16, 64, 256), (17, 65, 272), (28, 768, 768),
+          (31, 200, 4112), (32, 129, 1040), (33, 3072, 768), (45, 1024, 6144), (63, 384, 1536),
+          (64, 1536, 384), (64, 96, 8208)]
+# more rows, int8 only: 64x32 and 64x64 tiles, full and ragged
+INT8_SHAPES = [(65, 768, 3072), (200, 320, 2000), (349, 3072, 768), (1213, 768, 768),
+               (1024, 80, 1040)]
+
+
+def say(*a):
+    print(*a, flush=True)
+
+
+def rows(rng, m, k):
+    return (rng.standard_normal((m, k)) * np.exp(rng.uniform(-2, 2, (m, 1)))).astype(np.float32)
+
+
+@pytest.mark.parametrize("shape", SHAPES + INT8_SHAPES)
+def test_int8_bit_exact(gpu_ctx, shape):
+    m, k, n = shape
+    say(f"few-row int8 m={m} k={k} n={n}")
+    rng = np.random.default_rng(m + 3 * k + 5 * n)
+    a = rows(rng, m, k)
+    bT = (rng.standard_normal((n, k)) * 0.05).astype(np.float32)
+    bias = rng.standard_normal(n).astype(np.float32)
+    pb = T.PackB8VNNI(gpu_ctx, bT, k, n, bias)
+    got, (qa, rs) = T.matmul_host(gpu_ctx, a, pb)
+    _, q, sc, cs = O.pack_b8_vnni(bT, k, n)
+    want, qa_o, _, acc_o = O.matmul_vnni(a, q, cs, sc)
+    assert np.array_equal(qa[:, :k], qa_o)
+    assert np.array_equal(got, want)
+    # the raw accumulators, and bias + GELU in the epilogue
+    ldq = T.ldq_for(k)
+    dq, dacc = gpu_ctx.upload(qa), gpu_ctx.alloc(m * n * 4)
+    T.GemmU8S8I32(gpu_ctx, dacc, dq, ldq, pb, m)
+    gpu_ctx.sync()
+    assert np.array_equal(dacc.download(np.int32, (m, n)), acc_o)
+    got, _ = T.matmul_host(gpu_ctx, a, pb, act=_lib.RH_ACT_GELU)
+    assert np.array_equal(got, O.gelu_ref(want + bias))
+    # and the row-quantizing epilogues
+    st = rng.integers(1, 255, (m, ldq), dtype=np.uint8)
+    qo, rso, mx = gpu_ctx.upload(st), gpu_ctx.alloc(m * 4), gpu_ctx.alloc(m * 4)
+    ldo = T.ldq_for(n)
+    out = gpu_ctx.alloc(m * ldo)
+    T.LinearU8(gpu_ctx, dq, ldq, gpu_ctx.upload(rs), pb, m, _lib.RH_ACT_GELU, out, ldo, rso, mx)
+    gpu_ctx.sync()
+    pairs = [O.quantize_row_u8(r) for r in got]
+    assert np.array_equal(out.download(np.uint8, (m, ldo))[:, :n], np.stack([p[0] for p in pairs]))
+    assert np.array_equal(rso.download(np.float32, (m,)),
+                          np.array([p[1] for p in pairs], np.float32))
+    del qo
+
+
+@pytest.mark.parametrize("mode", ["w8", "fp32"])
+@pytest.mark.parametrize("terms", [1, 2])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_planes_against_float64(gpu_ctx, shape, terms, mode):
+    if mode == "fp32" and terms == 1:
+        pytest.skip("fp32 always takes two terms")
+    m, k, n = shape
+    say(f"few-row {mode} terms={terms} m={m} k={k} n={n}")
+    rng = np.random.default_rng(m + 3 * k + 5 * n + terms)
+    a = rows(rng, m, k)
+    bT = (rng.standard_normal((n, k)) * 0.05).astype(np.float32)
+    bias = rng.standard_normal(n).astype(np.float32)
+    gpu_ctx.set_option(_lib.RH_CTX_W8_TERMS, terms)
+    try:
+        if mode == "w8":
+            pb = T.PackB8(gpu_ctx, bT, k, n, bias)
+            q, sc, _ = pb.export()
+            w = q.astype(np.float64) * sc.astype(np.float64)[:, None]
+        else:
+            pb = T.PackB(gpu_ctx, bT, k, n, bias)
+            w = bT.astype(np.float64)
+        got = T.matmul_host(gpu_ctx, a, pb)
+    finally:
+        gpu_ctx.set_option(_lib.RH_CTX_W8_TERMS, 1)
+    a64 = a.astype(np.float64)
+    want = a64 @ w.T
+    # |error| <= sum |a||w| · (operand rounding + the fp32 sum's): one bf16 term
+    # is off by 2^-9 of a value at most, two by 2^-17 (and the dropped lo·lo
+    # product, and w's own split); K fp32 additions in any order by K · 2^-24
+    eps = 2.0 ** -9 if terms == 1 else 3 * 2.0 ** -17
+    bound = (np.abs(a64) @ np.abs(w).T) * (eps + k * 2.0 ** -24) + 1e-30
+    assert np.all(np.abs(got - want) <= bound)
+
+
+@pytest.mark.parametrize("mode", ["w8", "fp32"])
+@pytest.mark.parametrize("terms", [1, 2])
+@pytest.mark.parametrize("shape", [(1, 768, 768), (17, 40, 48), (33, 3072, 256), (45, 130, 512),
+                                   (200, 768, 272)])
+def test_planes_rows_equal_the_tiled_kernels(gpu_ctx, shape, terms, mode):
+    """A row's result does not depend on the rows computed with it: the same
+    bits as a forced tile of the tiled kernel."""
+    if mode == "fp32" and terms == 1:
+        pytest.skip("fp32 always takes two terms")
+    m, k, n = shape
+    say(f"few-row vs tiled {mode} terms={terms} m={m} k={k} n={n}")
+    rng = np.random.default_rng(m + k + n)
+    a = rows(rng, m, k)
+    bT = (rng.standard_normal((n, k)) * 0.05).astype(np.float32)
+    pb = T.PackedWeight(gpu_ctx, 1 if mode == "w8" else 0, bT, k, n,
+                        rng.standard_normal(n).astype(np.float32))
+    gpu_ctx.set_option(_lib.RH_CTX_W8_TERMS, terms)
+    try:
+        got = T.matmul_host(gpu_ctx, a, pb, act=_lib.RH_ACT_GELU)
+        gpu_ctx.set_option(_lib.RH_CTX_BF_TILE, 8)
+        want = T.matmul_host(gpu_ctx, a, pb, act=_lib.RH_ACT_GELU)
+    finally:
+        gpu_ctx.set_option(_lib.RH_CTX_BF_TILE, 0)
+        gpu_ctx.set_option(_lib.RH_CTX_W8_TERMS, 1)
+    assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("act", [_lib.RH_ACT_SWIGLU, _lib.RH_ACT_GEGLU, _lib.RH_ACT_GEGLU_ERF])
+@pytest.mark.parametrize("mode", [0, 1, 2])
+@pytest.mark.parametrize("shape", [(1, 768, 64), (17, 72, 1040), (45, 1024, 3072), (64, 768, 1152),
+                                   (100, 768, 3072)])
+def test_gated_equals_the_tiled_kernels(gpu_ctx, shape, mode, act):
+    """act(gate)·up in the epilogue: the same bits as a forced tile."""
+    m, k, i = shape
+    say(f"few-row gated mode={mode} act={act} m={m} k={k} i={i}")
+    rng = np.random.default_rng(m + k + i + act)
+    pg = T.PackedGated(gpu_ctx, mode, (rng.standard_normal((i, k)) * 0.05).astype(np.float32),
+                       (rng.standard_normal((i, k)) * 0.05).astype(np.float32), k, i)
+    da, dst = gpu_ctx.upload(rows(rng, m, k)), gpu_ctx.alloc(m * i * 4)
+    ldq = T.ldq_for(k)
+    qa, rs = gpu_ctx.alloc(m * ldq), gpu_ctx.alloc(m * 4)
+    option, tile = (_lib.RH_CTX_I8_TILE, 3) if mode == 2 else (_lib.RH_CTX_BF_TILE, 8)
+    out = []
+    for t in (0, tile):
+        gpu_ctx.set_option(option, t)
+        try:
+            T.Linear(gpu_ctx, dst, da, pg, m, act, qa if mode == 2 else None,
+                     ldq if mode == 2 else 0, rs if mode == 2 else None)
+            gpu_ctx.sync()
+        finally:
+            gpu_ctx.set_option(option, 0)
+        out.append(dst.download(np.float32, (m, i)))
+    assert np.array_equal(out[0], out[1])
