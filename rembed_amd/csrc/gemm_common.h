@@ -94,6 +94,44 @@ __device__ __forceinline__ void stage_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// Reductions over the wave, every lane getting the result: the butterfly over
+// l ^ 32, 16, 8, 4, 2, 1, each exchange a VALU operation (gfx950's
+// v_permlane32/16_swap, then DPP row rotations and quad permutes) instead of
+// an LDS-pipe ds_bpermute. After the exchanges with l ^ 32, 16 and 8 a rotation
+// by 4 brings the value of l ^ 4. The additions are those of the shuffle form
+// (a + b commutes), so the bits are too.
+template <class F>
+__device__ __forceinline__ float wave_butterfly(float v, F&& op) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef unsigned v2u __attribute__((ext_vector_type(2)));
+  {
+    const unsigned u = __float_as_uint(v);
+    const v2u r = __builtin_bit_cast(v2u, __builtin_amdgcn_permlane32_swap(u, u, false, false));
+    v = op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  }
+  {
+    const unsigned u = __float_as_uint(v);
+    const v2u r = __builtin_bit_cast(v2u, __builtin_amdgcn_permlane16_swap(u, u, false, false));
+    v = op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  }
+#define RH_DPP(ctrl)                                                                   \
+  v = op(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, 0xF, \
+                                                       0xF, true)))
+  RH_DPP(0x128);  // row_ror:8
+  RH_DPP(0x124);  // row_ror:4
+  RH_DPP(0x4E);   // quad_perm [2, 3, 0, 1]
+  RH_DPP(0xB1);   // quad_perm [1, 0, 3, 2]
+#undef RH_DPP
+#endif
+  return v;
+}
+__device__ __forceinline__ float wave_sum(float v) {
+  return wave_butterfly(v, [](float a, float b) { return a + b; });
+}
+__device__ __forceinline__ float wave_max(float v) {
+  return wave_butterfly(v, [](float a, float b) { return fmaxf(a, b); });
+}
+
 // erf-GELU with exactly the float32 operation sequence of the reference's
 // geluScalar (internal/tensor/tensor.go:508-538; exp body fastmath.go:93-109).
 // The library is compiled with -ffp-contract=off, so no FMA is formed here.

@@ -13,16 +13,6 @@ namespace {
 
 constexpr int kRows = 4;  // 256 threads = 4 waves = 4 rows
 
-__device__ __forceinline__ float wsum(float v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
-__device__ __forceinline__ float wmax(float v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
-}
 __device__ __forceinline__ uint8_t qbyte(float v, float inv) {
   int q = (int)rintf(v * inv) + 128;
   return (uint8_t)(q < 0 ? 0 : (q > 255 ? 255 : q));
@@ -115,7 +105,7 @@ __global__ __launch_bounds__(256) void rms_residual_kernel(RmsArgs p) {
       ss += (w[e][0] * w[e][0] + w[e][1] * w[e][1]) + (w[e][2] * w[e][2] + w[e][3] * w[e][3]);
     }
     if (p.post_g) {
-      const float inv = rms_inv(wsum(ss), H, p.eps);
+      const float inv = rms_inv(wave_sum(ss), H, p.eps);
 #pragma unroll
       for (int e = 0; e < V; e++) {
         const int j = (lane + 64 * e) * 4;
@@ -141,7 +131,7 @@ __global__ __launch_bounds__(256) void rms_residual_kernel(RmsArgs p) {
     float s = 0.0f;  // lanes past H hold zeros
 #pragma unroll
     for (int e = 0; e < V; e++) s += (v[e][0] + v[e][1]) + (v[e][2] + v[e][3]);
-    mean = wsum(s) / (float)H;
+    mean = wave_sum(s) / (float)H;
     float s2 = 0.0f;
 #pragma unroll
     for (int e = 0; e < V; e++) {
@@ -151,13 +141,13 @@ __global__ __launch_bounds__(256) void rms_residual_kernel(RmsArgs p) {
         s2 += (d[0] * d[0] + d[1] * d[1]) + (d[2] * d[2] + d[3] * d[3]);
       }
     }
-    inv = 1.0f / sqrtf(wsum(s2) / (float)H + p.eps);
+    inv = 1.0f / sqrtf(wave_sum(s2) / (float)H + p.eps);
   } else {
     float ss = 0.0f;
 #pragma unroll
     for (int e = 0; e < V; e++)
       ss += (v[e][0] * v[e][0] + v[e][1] * v[e][1]) + (v[e][2] * v[e][2] + v[e][3] * v[e][3]);
-    inv = rms_inv(wsum(ss), H, p.eps);
+    inv = rms_inv(wave_sum(ss), H, p.eps);
   }
   float mx = 0.0f;
 #pragma unroll
@@ -182,7 +172,7 @@ __global__ __launch_bounds__(256) void rms_residual_kernel(RmsArgs p) {
     }
   }
   if (p.qa) {  // QuantizeRowU8 (pack_vnni.go:85-117) of the normalized row
-    mx = wmax(mx);
+    mx = wave_max(mx);
     float scale = mx / 127.0f;
     if (scale == 0.0f) scale = 1.0f;
     const float qinv = 1.0f / scale;
@@ -274,7 +264,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(
     float ss = 0.0f;
 #pragma unroll
     for (int e = 0; e < 2; e++) ss += x1[it][e] * x1[it][e] + x2[it][e] * x2[it][e];
-    const float inv = rms_inv(wsum(ss), dh, eps);
+    const float inv = rms_inv(wave_sum(ss), dh, eps);
     const int p = pos[row];
     const float* c = cos_t + (size_t)p * half;
     const float* sn = sin_t + (size_t)p * half;

@@ -153,3 +153,28 @@ def test_gated_equals_the_tiled_kernels(gpu_ctx, shape, mode, act):
             gpu_ctx.set_option(option, 0)
         out.append(dst.download(np.float32, (m, i)))
     assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("n", [384, 768, 1024, 1028, 2048])
+def test_row_kernels_few_and_many_rows_agree(gpu_ctx, n):
+    """LayerNorm and QuantizeRowU8 of the same rows in a call of one row, of the
+    most rows that run one per wave (2048) and of one more: the same bits, and
+    the quantizer's equal the oracle's."""
+    say(f"row kernels n={n}")
+    rng = np.random.default_rng(n)
+    m = 2049
+    x = rows(rng, m, n)
+    g = gpu_ctx.upload((1 + 0.1 * rng.standard_normal(n)).astype(np.float32))
+    b = gpu_ctx.upload(rng.standard_normal(n).astype(np.float32))
+    ln, qs = {}, {}
+    for k in (1, 2048, m):
+        dx = gpu_ctx.upload(x[:k])
+        _lib.check(_lib.lib.rh_layernorm(gpu_ctx.h, dx.ptr, g.ptr, b.ptr, k, n, 1e-12))
+        da, dq, ds = gpu_ctx.upload(x[:k]), gpu_ctx.alloc(k * n), gpu_ctx.alloc(k * 4)
+        T.QuantizeRowsU8(gpu_ctx, da, k, n, dq, n, ds)
+        gpu_ctx.sync()
+        ln[k] = dx.download(np.float32, (k, n))
+        qs[k] = dq.download(np.uint8, (k, n))
+    assert np.array_equal(ln[2048][:1], ln[1]) and np.array_equal(ln[m][:2048], ln[2048])
+    assert np.array_equal(qs[2048][:1], qs[1]) and np.array_equal(qs[m][:2048], qs[2048])
+    assert np.array_equal(qs[m], np.stack([O.quantize_row_u8(r)[0] for r in x]))
