@@ -18,22 +18,23 @@
 namespace rh {
 
 constexpr int kAttnQ = 128;   // queries per workgroup (4 waves x 32)
-constexpr int kAttnKV = 64;   // keys per LDS block
+constexpr int kAttnKV = 64;   // keys per LDS block of one-term products
 
-// 8 consecutive activations as floats, from fp32 (two 16-byte loads) or bf16
-// (one 16-byte load; widening is exact).
-__device__ __forceinline__ void load8(const float* src, float (&x)[8]) {
-  const v4f a = reinterpret_cast<const v4f*>(src)[0], b = reinterpret_cast<const v4f*>(src)[1];
-#pragma unroll
-  for (int e = 0; e < 4; e++) {
-    x[e] = a[e];
-    x[4 + e] = b[e];
-  }
+// 8 consecutive fp32 values, and their bf16 split hi = bf16(x), lo = bf16(x - hi).
+struct F8 {
+  v4f a, b;
+};
+__device__ __forceinline__ F8 load8(const float* src) {
+  return {reinterpret_cast<const v4f*>(src)[0], reinterpret_cast<const v4f*>(src)[1]};
 }
-__device__ __forceinline__ void load8(const __bf16* src, float (&x)[8]) {
-  const v8bf a = *reinterpret_cast<const v8bf*>(src);
+template <bool LO>
+__device__ __forceinline__ void split8(const F8& x, v8bf& hi, v8bf& lo) {
 #pragma unroll
-  for (int e = 0; e < 8; e++) x[e] = (float)a[e];
+  for (int e = 0; e < 8; e++) {
+    const float v = e < 4 ? x.a[e] : x.b[e - 4];
+    hi[e] = (__bf16)v;
+    if constexpr (LO) lo[e] = (__bf16)(v - (float)hi[e]);
+  }
 }
 
 // Visible keys of query qi (text-local): [klo, khi]. Keys past the text,
@@ -50,16 +51,21 @@ __device__ __forceinline__ void attn_key_range(const AttnArgs& p, int qi, int le
   }
 }
 
-// Online-softmax step for one 64-key block held as S^T tiles (lane: query
+// Online-softmax step for one key block held as S^T tiles (lane: query
 // fr, keys key0 + t2*32 + i*8 + fg*4 + j in register t2, i*4 + j). Scores
 // go to log2 units through cs = scale·log2 e, folded into the exponent:
 // the block max of s·cs is max(s)·cs exactly (rounding is monotonic and
 // cs > 0), and p = 2^fma(s, cs, -m). `masked` (uniform over the wave)
 // applies the per-key range test. P = 2^(s·cs - mref) against a reference
-// that moves only when a block's max exceeds it by more than 8: P stays
-// <= 256 (no overflow in fp32), and the running output is rescaled (by the
-// returned alpha, when `rescale`) only on those moves. sc becomes P.
-__device__ __forceinline__ float attn_softmax_block(v16f (&sc)[2], int key0, int fg, int klo,
+// that moves only when a block's max exceeds it by more than kSlack: P stays
+// <= 2^kSlack (no overflow in fp32), and the running output is rescaled (by
+// the returned alpha, when `rescale`) only on those moves. sc becomes P.
+// The fp32-grade products on 32-key blocks take a slack of 1: a query's largest P is then split
+// (nearly) exactly, and their error is below that of 64-key blocks with a slack
+// of 8 (24 texts of 33..512, head dim 64: 6.2e-6 against 6.3e-6 of the output)
+// for 1-2 % of the time.
+template <int NT, int kSlack>
+__device__ __forceinline__ float attn_softmax_block(v16f (&sc)[NT], int key0, int fg, int klo,
                                                     int khi, bool masked, float cs,
                                                     float& mref, float& lrun, bool& rescale) {
   // One uniform branch around the whole mask (a per-element condition is
@@ -71,7 +77,7 @@ __device__ __forceinline__ float attn_softmax_block(v16f (&sc)[2], int key0, int
     const unsigned span = (unsigned)(khi - klo);
     const int base = key0 + fg * 4 - klo;
 #pragma unroll
-    for (int t2 = 0; t2 < 2; t2++)
+    for (int t2 = 0; t2 < NT; t2++)
 #pragma unroll
       for (int i = 0; i < 4; i++)
 #pragma unroll
@@ -82,14 +88,14 @@ __device__ __forceinline__ float attn_softmax_block(v16f (&sc)[2], int key0, int
   }
   float smax = -INFINITY;
 #pragma unroll
-  for (int t2 = 0; t2 < 2; t2++)
+  for (int t2 = 0; t2 < NT; t2++)
 #pragma unroll
     for (int e = 0; e < 16; e++) smax = fmaxf(smax, sc[t2][e]);
   smax = fmaxf(smax, __shfl_xor(smax, 32, 64));
   const float mloc = smax * cs;
-  // -inf + 8 = -inf: a lane's first visible key always moves the reference
+  // -inf + slack = -inf: a lane's first visible key always moves the reference
   // (alpha = 2^-inf = 0 then); a lane with no visible key keeps -inf.
-  const bool up = mloc > mref + 8.0f;
+  const bool up = mloc > mref + (float)kSlack;
   rescale = __any(up);
   float alpha = 1.0f;
   if (up) {
@@ -99,7 +105,7 @@ __device__ __forceinline__ float attn_softmax_block(v16f (&sc)[2], int key0, int
   const float m = mref == -INFINITY ? 0.0f : mref;  // all-masked lanes: every p = 0
   float psum = 0.0f;
 #pragma unroll
-  for (int t2 = 0; t2 < 2; t2++)
+  for (int t2 = 0; t2 < NT; t2++)
 #pragma unroll
     for (int e = 0; e < 16; e++) {
       const float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[t2][e], cs, -m));
@@ -136,12 +142,13 @@ __device__ __forceinline__ void attn_split8(const v16f& s, int base, v8bf& ph, v
 // with cs = log2 e. Lane layout as attn_softmax_block (query qi; keys key0 +
 // t2*32 + i*8 + fg*4 + j). Relative positions outside the table belong to
 // masked keys or unstored queries and are clamped into it.
-__device__ __forceinline__ void attn_rel_bias(const AttnArgs& p, v16f (&sc)[2], int h, int qi,
+template <int NT>
+__device__ __forceinline__ void attn_rel_bias(const AttnArgs& p, v16f (&sc)[NT], int h, int qi,
                                               int key0, int fg) {
   const int c = p.rel_center;
   const float* rb = p.rel_bias + (size_t)h * (2 * c + 1) + c;
 #pragma unroll
-  for (int t2 = 0; t2 < 2; t2++)
+  for (int t2 = 0; t2 < NT; t2++)
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
@@ -212,205 +219,28 @@ __device__ __forceinline__ void attn_store_rows(const AttnArgs& p, const v16f (&
   }
 }
 
-template <int DH, int PREC, typename TIn>
-__global__ __launch_bounds__(256) void attention_kernel(AttnArgs p) {
-  const TIn* qkv = static_cast<const TIn*>(p.qkv);
-  constexpr int T = PREC == 3 ? 2 : 1;        // bf16 planes per operand
-  constexpr int KS = DH / 16;                 // k-steps over dh
-  constexpr int DT = DH / 32;                 // 32-wide d tiles of O^T
-  constexpr int kK = kAttnKV * DH * 2;        // bytes of one K plane
-  constexpr int kV = DH * kAttnKV * 2;        // bytes of one V^T plane
-  // XOR swizzle of 16-byte chunks inside a K row, kept inside the row
-  // (a row holds DH/8 chunks: 4 for dh 32, 8 or more otherwise).
-  constexpr int kSwz = DH / 8 >= 8 ? 7 : DH / 8 - 1;
-  constexpr int kOut = 4 * 32 * (DH + 4) * 4;  // output staging (attn_store_rows)
-  __shared__ __attribute__((aligned(16))) uint8_t lds[T * (kK + kV) > kOut ? T * (kK + kV) : kOut];
-  uint8_t* sK = lds;
-  uint8_t* sV = lds + T * kK;
-
-  int b, h, qb;
-  if (!attn_block(p, b, h, qb)) return;
-  const int r0 = p.cu[b], len = p.cu[b + 1] - r0;
-  const int q0 = qb * kAttnQ;
-  if (q0 >= len) return;
-  const int kvh = h / (p.heads / p.kv_heads);
-
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int fr = lane & 31, fg = lane >> 5;
-  const int qi = q0 + wave * 32 + fr;  // this lane's query (text-local)
-
-  // Q fragments (B operand of S^T): lane (query fr, half fg) holds
-  // Q[q][s*16 + fg*8 + e].
-  v8bf qh[KS], ql[KS];
-  {
-    // rows past the text read its last row; their outputs are not stored
-    const TIn* qrow = qkv + (size_t)(r0 + (qi < len ? qi : len - 1)) * p.ldqkv + p.q_off + h * DH;
-#pragma unroll
-    for (int s = 0; s < KS; s++) {
-      float xq[8];
-      load8(qrow + s * 16 + fg * 8, xq);
-#pragma unroll
-      for (int e = 0; e < 8; e++) {
-        const __bf16 hi = (__bf16)xq[e];
-        qh[s][e] = hi;
-        if constexpr (PREC == 3) ql[s][e] = (__bf16)(xq[e] - (float)hi);
-      }
-    }
-  }
-
-  v16f o[DT];
-#pragma unroll
-  for (int t = 0; t < DT; t++)
-#pragma unroll
-    for (int e = 0; e < 16; e++) o[t][e] = 0.0f;
-  float mrun = -INFINITY, lrun = 0.0f;
-  const float cs = p.scale * 1.44269504088896341f;  // scores in log2 units
-  int klo, khi;
-  attn_key_range(p, qi, len, klo, khi);
-
-  // Key blocks this workgroup's queries can see: causal stops after the
-  // last query; a window bounds both ends (|i - j| < window).
-  int kb_lo = 0, kb_hi = (len + kAttnKV - 1) / kAttnKV;
-  const int qlast = min(q0 + kAttnQ, len) - 1;
-  if (p.causal) kb_hi = min(kb_hi, qlast / kAttnKV + 1);
-  if (p.window > 0) {
-    kb_lo = max(0, q0 - p.window + 1) / kAttnKV;
-    kb_hi = min(kb_hi, (qlast + p.window - 1) / kAttnKV + 1);
-  }
-  for (int kb = kb_lo; kb < kb_hi; kb++) {
-    const int key0 = kb * kAttnKV;
-    __syncthreads();  // previous block's LDS reads are done
-    // Stage K (row-major [key][d], swizzled 16B chunks) and V^T ([d][key]).
-    constexpr int kChunksPerRow = DH / 8;
-    for (int it = tid; it < kAttnKV * kChunksPerRow; it += 256) {
-      const int key = it / kChunksPerRow, ch = it % kChunksPerRow;
-      const int kg = key0 + key;
-      // Unconditional loads from a clamped in-text row; keys past the text
-      // are zeroed after the loads (and masked out of the softmax below).
-      const bool kok = kg < len;
-      const size_t rowk = (size_t)(r0 + (kok ? kg : len - 1)) * p.ldqkv;
-      float kx[8], vx[8];
-      load8(qkv + rowk + p.k_off + kvh * DH + ch * 8, kx);
-      load8(qkv + rowk + p.v_off + kvh * DH + ch * 8, vx);
-#pragma unroll
-      for (int e = 0; e < 8; e++) {
-        kx[e] = kok ? kx[e] : 0.0f;
-        vx[e] = kok ? vx[e] : 0.0f;
-      }
-      v8bf khi, klo;
-#pragma unroll
-      for (int e = 0; e < 8; e++) {
-        const __bf16 hi = (__bf16)kx[e];
-        khi[e] = hi;
-        if constexpr (PREC == 3) klo[e] = (__bf16)(kx[e] - (float)hi);
-      }
-      const int koff = key * (DH * 2) + ((ch ^ (key & kSwz)) << 4);
-      *reinterpret_cast<v8bf*>(sK + koff) = khi;
-      if constexpr (PREC == 3) *reinterpret_cast<v8bf*>(sK + kK + koff) = klo;
-#pragma unroll
-      for (int e = 0; e < 8; e++) {
-        const int d = ch * 8 + e;
-        const int voff = d * (kAttnKV * 2) + (((key >> 3) ^ (d & 7)) << 4) + ((key & 7) << 1);
-        const __bf16 hi = (__bf16)vx[e];
-        *reinterpret_cast<__bf16*>(sV + voff) = hi;
-        if constexpr (PREC == 3)
-          *reinterpret_cast<__bf16*>(sV + kV + voff) = (__bf16)(vx[e] - (float)hi);
-      }
-    }
-    __syncthreads();
-
-    // S^T for the two 32-key tiles of this block.
-    v16f sc[2];
-#pragma unroll
-    for (int t2 = 0; t2 < 2; t2++) {
-#pragma unroll
-      for (int e = 0; e < 16; e++) sc[t2][e] = 0.0f;
-      const int key = t2 * 32 + fr;
-#pragma unroll
-      for (int s = 0; s < KS; s++) {
-        const int ch = 2 * s + fg;
-        const int koff = key * (DH * 2) + ((ch ^ (key & kSwz)) << 4);
-        const v8bf kh = *reinterpret_cast<const v8bf*>(sK + koff);
-        sc[t2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kh, qh[s], sc[t2], 0, 0, 0);
-        if constexpr (PREC == 3) {
-          const v8bf kl = *reinterpret_cast<const v8bf*>(sK + kK + koff);
-          sc[t2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kh, ql[s], sc[t2], 0, 0, 0);
-          sc[t2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kl, qh[s], sc[t2], 0, 0, 0);
-        }
-      }
-    }
-    // Scale, mask, online softmax; the output is rescaled only when some
-    // query's reference max moved.
-    const bool masked = __any(key0 < klo || key0 + kAttnKV - 1 > khi);
-    bool rescale;
-    if (p.rel_bias) attn_rel_bias(p, sc, h, qi, key0, fg);
-    const float alpha = attn_softmax_block(sc, key0, fg, klo, khi, masked,
-                                           p.rel_bias ? 1.44269504088896341f : cs, mrun,
-                                           lrun, rescale);
-    if (rescale) {
-#pragma unroll
-      for (int t = 0; t < DT; t++)
-#pragma unroll
-        for (int e = 0; e < 16; e++) o[t][e] *= alpha;
-    }
-
-    // O^T += V^T · P^T over 4 chunks of 16 keys. Chunk kc, lane half g,
-    // element e <-> key kc*16 + (e/4)*8 + g*4 + e%4 = register
-    // sc[kc/2][(kc%2)*8 + e].
-#pragma unroll
-    for (int kc = 0; kc < 4; kc++) {
-      v8bf ph, pl;
-      if constexpr (PREC == 3) {
-        attn_split8(sc[kc >> 1], (kc & 1) * 8, ph, pl);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; e++) ph[e] = (__bf16)sc[kc >> 1][(kc & 1) * 8 + e];
-      }
-#pragma unroll
-      for (int t = 0; t < DT; t++) {
-        const int d = t * 32 + fr;
-        const int base = d * (kAttnKV * 2);
-        const int c0 = 2 * kc, c1 = 2 * kc + 1;
-        const int off0 = base + ((c0 ^ (d & 7)) << 4) + fg * 8;
-        const int off1 = base + ((c1 ^ (d & 7)) << 4) + fg * 8;
-        v8bf vh;
-        {
-          typedef short v4s __attribute__((ext_vector_type(4)));
-          const v4s a = *reinterpret_cast<const v4s*>(sV + off0);
-          const v4s c = *reinterpret_cast<const v4s*>(sV + off1);
-          v8s w = {a[0], a[1], a[2], a[3], c[0], c[1], c[2], c[3]};
-          vh = __builtin_bit_cast(v8bf, w);
-        }
-        o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vh, ph, o[t], 0, 0, 0);
-        if constexpr (PREC == 3) {
-          typedef short v4s __attribute__((ext_vector_type(4)));
-          const v4s a = *reinterpret_cast<const v4s*>(sV + kV + off0);
-          const v4s c = *reinterpret_cast<const v4s*>(sV + kV + off1);
-          v8s w = {a[0], a[1], a[2], a[3], c[0], c[1], c[2], c[3]};
-          const v8bf vl = __builtin_bit_cast(v8bf, w);
-          o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vh, pl, o[t], 0, 0, 0);
-          o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vl, ph, o[t], 0, 0, 0);
-        }
-      }
-    }
-  }
-
-  const float ltot = lrun + __shfl_xor(lrun, 32, 64);
-  // rows past the text divide by 1 (their values are never stored)
-  const float inv = 1.0f / (qi < len ? ltot : 1.0f);
-  __syncthreads();  // every wave's reads of the last key block are done
-  attn_store_rows<DH>(p, o, inv, lds, wave, lane, r0, q0 + wave * 32, len, h);
-}
-
-// ---- bf16 operands, pipelined --------------------------------------------------
-// The same algorithm and fragment layouts for bf16 q|k|v rows, with the key
-// blocks double-buffered: while a block is multiplied, the next block's K
-// and V rows stream into LDS by global_load_lds_dwordx4.
+// ---- the pipelined kernel -------------------------------------------------------
+// Key blocks are double-buffered in LDS: while a block is multiplied, the next
+// block's K and V rows are on their way. bf16 rows (T 1) and bf16 hi/lo planes
+// (T 2: three products per MFMA step) stream in by global_load_lds_dwordx4;
+// fp32 rows (F32) are loaded into registers before a block's products, split
+// and stored after them.
 //
-// K block: [64 keys][DH] bf16, 16-byte chunk c of row r at slot c ^ kswz(r)
+// What bounds it: the softmax's VALU work and the matrix cores in turn (a wave's
+// scores, softmax and P·V depend on each other), so it lives on waves per SIMD.
+// Three-term blocks therefore hold 32 keys at head dims 128 and up (and of fp32
+// rows at 64): two 64-KiB workgroups per CU at head dim 128, where 64 keys left
+// one. Measured on MI355X
+// (µs; before: fp32 rows staged between two barriers, V transposed by 2-byte
+// stores; planes with 64-key blocks):
+//   fp32 rows, 24 texts of 33..512, 16 heads of 64            100 -> 61
+//   fp32 rows, 12 causal texts of 97..512, 16/8 heads of 128  134 -> 60
+//   fp32 rows, 6 texts of 300..2048, 3/1 heads of 256        1265 -> 470
+//   planes, the head dim 128 case                            62.8 -> 54.4
+//
+// K block: [KV keys][DH] bf16, 16-byte chunk c of row r at slot c ^ kswz(r)
 // (16 consecutive rows of one fragment read land in 16 distinct bank
-// groups). V block: [64 keys][DH] bf16 as well, 64-byte pieces swizzled by
+// groups). V block: [KV keys][DH] bf16 as well, 64-byte pieces swizzled by
 // attn_vswz; the PV products read it transposed (ds_read_b64_tr_b16), so
 // each lane's V^T fragment holds the keys in the order its P^T registers
 // do (see below).
@@ -443,15 +273,16 @@ __device__ __forceinline__ int attn_vswz(int r) {
   return DH == 64 ? (r >> 1) & 1 : DH >= 128 ? r & 3 : 0;
 }
 
-template <int DH, int T>
-__global__ __launch_bounds__(256) void attention_bf16_kernel(AttnArgs p) {
+template <int DH, int T, int KV, bool F32, int MINW>
+__global__ __launch_bounds__(256, MINW) void attention_bf16_kernel(AttnArgs p) {
   const __bf16* qkv = static_cast<const __bf16*>(p.qkv);
-  const __bf16* qkv_lo = static_cast<const __bf16*>(p.qkv_lo);  // T == 2
-  constexpr int KS = DH / 16, DT = DH / 32;
+  const __bf16* qkv_lo = static_cast<const __bf16*>(p.qkv_lo);  // T == 2, !F32
+  const float* qkv_f = static_cast<const float*>(p.qkv);        // F32
+  constexpr int KS = DH / 16, DT = DH / 32, NT = KV / 32;
   constexpr int kRowB = DH * 2;               // bytes of one K row
-  constexpr int kKB = kAttnKV * kRowB;        // K block bytes
+  constexpr int kKB = KV * kRowB;             // K block bytes
   constexpr int kStage = 2 * kKB * T;         // K + V (same size), per plane
-  constexpr int kKLoads = kKB / (4 * 1024);   // DMA instructions per wave per block
+  constexpr int kKLoads = kKB / (4 * 1024);   // 16-byte chunks per thread and block
   static_assert(kKLoads >= 1 && kKB % 4096 == 0, "K block must split into 4 waves x 1 KiB");
   constexpr int kOut = 4 * 32 * (DH + 4) * 4;  // output staging (attn_store_rows)
   __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * kStage > kOut ? 2 * kStage : kOut];
@@ -467,59 +298,78 @@ __global__ __launch_bounds__(256) void attention_bf16_kernel(AttnArgs p) {
   const int fr = lane & 31, fg = lane >> 5;
   const int qi = q0 + wave * 32 + fr;
 
-  // Q fragments (B operand of S^T), straight from the bf16 rows.
+  // Q fragments (B operand of S^T): lane (query fr, half fg) holds
+  // Q[q][s*16 + fg*8 + e]. Rows past the text read its last row; their
+  // outputs are not stored.
   v8bf qf[KS], ql[KS];
   {
     const size_t qo = (size_t)(r0 + (qi < len ? qi : len - 1)) * p.ldqkv + p.q_off + h * DH;
 #pragma unroll
     for (int s = 0; s < KS; s++) {
+      if constexpr (F32) {
+        split8<T == 2>(load8(qkv_f + qo + s * 16 + fg * 8), qf[s], ql[s]);
+        continue;
+      }
       qf[s] = *reinterpret_cast<const v8bf*>(qkv + qo + s * 16 + fg * 8);
       if constexpr (T == 2) ql[s] = *reinterpret_cast<const v8bf*>(qkv_lo + qo + s * 16 + fg * 8);
     }
   }
 
-  // K DMA: this lane's slot in each of its 1 KiB blocks -> (row, chunk).
-  int k_row[kKLoads], k_chunk[kKLoads];
+  // This thread's 16-byte slots of a K or V block: slot off of plane t lies at
+  // t * 2 * kKB (+ kKB for V) + off; it holds row k_row, logical chunk k_chunk
+  // (K's swizzle) or v_chunk (V's swizzle, on 64-byte pieces of 4 chunks).
+  int k_row[kKLoads], k_chunk[kKLoads], v_chunk[kKLoads];
 #pragma unroll
   for (int j = 0; j < kKLoads; j++) {
     const int off = (wave * kKLoads + j) * 1024 + lane * 16;
     k_row[j] = off / kRowB;
     k_chunk[j] = ((off % kRowB) >> 4) ^ attn_kswz<DH>(k_row[j]);
+    v_chunk[j] = ((off % kRowB) >> 4) ^ (4 * attn_vswz<DH>(k_row[j]));
   }
-  // plane t of a stage: K at t * 2 * kKB, V^T right after it
   const size_t kvo = (size_t)p.k_off + kvh * DH, vvo = (size_t)p.v_off + kvh * DH;
-  auto issue_k = [&](int kb, int buf) {
+  // bf16 rows: DMA into the other buffer, waited for by the block's barrier
+  auto issue = [&](int kb, int buf) {
 #pragma unroll
     for (int t = 0; t < T; t++) {
       uint8_t* sK = lds + buf * kStage + t * 2 * kKB;
-      const __bf16* kbase = (t ? qkv_lo : qkv) + kvo;
+      const __bf16* base = t ? qkv_lo : qkv;
 #pragma unroll
       for (int j = 0; j < kKLoads; j++) {
-        const int kg = kb * kAttnKV + k_row[j];
-        const __bf16* src =
-            kbase + (size_t)(r0 + (kg < len ? kg : len - 1)) * p.ldqkv + k_chunk[j] * 8;
-        lds_dma16(src, sK + (wave * kKLoads + j) * 1024);
+        const int kg = kb * KV + k_row[j];
+        const __bf16* row = base + (size_t)(r0 + (kg < len ? kg : len - 1)) * p.ldqkv;
+        lds_dma16(row + kvo + k_chunk[j] * 8, sK + (wave * kKLoads + j) * 1024);
+        lds_dma16(row + vvo + v_chunk[j] * 8, sK + kKB + (wave * kKLoads + j) * 1024);
       }
     }
   };
-  // V DMA: the K slots with the V swizzle on 64-byte pieces (4 chunks)
-  int v_chunk[kKLoads];
+  // fp32 rows: loads into registers before a block's products, the split and
+  // the LDS stores after them. Keys past the text become zeros (their scores
+  // are masked; an infinity in the text's last row must not reach them).
+  F8 kx[F32 ? kKLoads : 1], vx[F32 ? kKLoads : 1];
+  auto fetch = [&](int kb) {
 #pragma unroll
-  for (int j = 0; j < kKLoads; j++) {
-    const int off = (wave * kKLoads + j) * 1024 + lane * 16;
-    v_chunk[j] = ((off % kRowB) >> 4) ^ (4 * attn_vswz<DH>(k_row[j]));
-  }
-  auto issue_v = [&](int kb, int buf) {
+    for (int j = 0; j < kKLoads; j++) {
+      const int kg = kb * KV + k_row[j];
+      const float* row = qkv_f + (size_t)(r0 + (kg < len ? kg : len - 1)) * p.ldqkv;
+      kx[j] = load8(row + kvo + k_chunk[j] * 8);
+      vx[j] = load8(row + vvo + v_chunk[j] * 8);
+    }
+  };
+  auto stash = [&](int kb, int buf) {
 #pragma unroll
-    for (int t = 0; t < T; t++) {
-      uint8_t* sV = lds + buf * kStage + t * 2 * kKB + kKB;
-      const __bf16* vbase = (t ? qkv_lo : qkv) + vvo;
-#pragma unroll
-      for (int j = 0; j < kKLoads; j++) {
-        const int kg = kb * kAttnKV + k_row[j];
-        lds_dma16(vbase + (size_t)(r0 + (kg < len ? kg : len - 1)) * p.ldqkv + v_chunk[j] * 8,
-                  sV + (wave * kKLoads + j) * 1024);
+    for (int j = 0; j < kKLoads; j++) {
+      if (kb * KV + k_row[j] >= len) {
+        kx[j] = F8{v4f{0.0f, 0.0f, 0.0f, 0.0f}, v4f{0.0f, 0.0f, 0.0f, 0.0f}};
+        vx[j] = kx[j];
       }
+      uint8_t* at = lds + buf * kStage + (wave * kKLoads + j) * 1024 + lane * 16;
+      v8bf hi, lo;
+      split8<T == 2>(kx[j], hi, lo);
+      *reinterpret_cast<v8bf*>(at) = hi;
+      if constexpr (T == 2) *reinterpret_cast<v8bf*>(at + 2 * kKB) = lo;
+      split8<T == 2>(vx[j], hi, lo);
+      *reinterpret_cast<v8bf*>(at + kKB) = hi;
+      if constexpr (T == 2) *reinterpret_cast<v8bf*>(at + 3 * kKB) = lo;
     }
   };
   // PV A fragments (lane (fr, g): dim 32t + fr of keys 16kc + 8(e/4) + 4g +
@@ -546,45 +396,49 @@ __global__ __launch_bounds__(256) void attention_bf16_kernel(AttnArgs p) {
   int klo, khi;
   attn_key_range(p, qi, len, klo, khi);
 
-  int kb_lo = 0, kb_hi = (len + kAttnKV - 1) / kAttnKV;
+  int kb_lo = 0, kb_hi = (len + KV - 1) / KV;
   const int qlast = min(q0 + kAttnQ, len) - 1;
-  if (p.causal) kb_hi = min(kb_hi, qlast / kAttnKV + 1);
+  if (p.causal) kb_hi = min(kb_hi, qlast / KV + 1);
   if (p.window > 0) {
-    kb_lo = max(0, q0 - p.window + 1) / kAttnKV;
-    kb_hi = min(kb_hi, (qlast + p.window - 1) / kAttnKV + 1);
+    kb_lo = max(0, q0 - p.window + 1) / KV;
+    kb_hi = min(kb_hi, (qlast + p.window - 1) / KV + 1);
   }
   // every query sees every key of its text: the only mask is the text's end
   const bool text_mask = !p.causal && p.window <= 0;
 
-  issue_k(kb_lo, 0);
-  issue_v(kb_lo, 0);
+  if constexpr (F32) {
+    fetch(kb_lo);
+    stash(kb_lo, 0);
+  } else {
+    issue(kb_lo, 0);
+  }
   __syncthreads();  // waits for the DMA (vmcnt)
 
   for (int kb = kb_lo; kb < kb_hi; kb++) {
     const int buf = (kb - kb_lo) & 1;
     const bool next = kb + 1 < kb_hi;
     if (next) {
-      issue_k(kb + 1, buf ^ 1);
-      issue_v(kb + 1, buf ^ 1);
+      if constexpr (F32) fetch(kb + 1);
+      else issue(kb + 1, buf ^ 1);
     }
     const uint8_t* sK = lds + buf * kStage;
     const uint8_t* sV = sK + kKB;
     const uint8_t* sKl = sK + 2 * kKB;  // T == 2: the lo planes
     const uint8_t* sVl = sKl + kKB;
-    const int key0 = kb * kAttnKV;
+    const int key0 = kb * KV;
 
     // A wave whose queries all lie past the text only helps stage blocks.
     if (q0 + wave * 32 < len) {
-    // S^T for the two 32-key tiles, the two accumulation chains interleaved.
-    v16f sc[2];
+    // S^T for the 32-key tiles, their accumulation chains interleaved.
+    v16f sc[NT];
 #pragma unroll
-    for (int t2 = 0; t2 < 2; t2++)
+    for (int t2 = 0; t2 < NT; t2++)
 #pragma unroll
       for (int e = 0; e < 16; e++) sc[t2][e] = 0.0f;
 #pragma unroll
     for (int s = 0; s < KS; s++)
 #pragma unroll
-      for (int t2 = 0; t2 < 2; t2++) {
+      for (int t2 = 0; t2 < NT; t2++) {
         const int kr = t2 * 32 + fr;
         const int ko = kr * kRowB + (((2 * s + fg) ^ attn_kswz<DH>(kr)) << 4);
         const v8bf kf = *reinterpret_cast<const v8bf*>(sK + ko);
@@ -600,12 +454,12 @@ __global__ __launch_bounds__(256) void attention_bf16_kernel(AttnArgs p) {
     // scores (k-element 0 of a mask fragment times q-element 0 = 1; every
     // other product is 0 * 0) and +0 to the rest, which leaves those sums
     // as they were, in place of a compare and select per score.
-    const bool key_tail = key0 + kAttnKV > len;
+    const bool key_tail = key0 + KV > len;
     if (text_mask && key_tail) {
       const v8bf q1 = {(__bf16)(fg == 0 ? 1.0f : 0.0f), (__bf16)0.0f, (__bf16)0.0f, (__bf16)0.0f,
                        (__bf16)0.0f, (__bf16)0.0f, (__bf16)0.0f, (__bf16)0.0f};
 #pragma unroll
-      for (int t2 = 0; t2 < 2; t2++) {
+      for (int t2 = 0; t2 < NT; t2++) {
         const bool past = key0 + t2 * 32 + fr >= len;
         const v8bf km = {(__bf16)(fg == 0 && past ? -INFINITY : 0.0f), (__bf16)0.0f, (__bf16)0.0f,
                          (__bf16)0.0f, (__bf16)0.0f, (__bf16)0.0f, (__bf16)0.0f, (__bf16)0.0f};
@@ -616,12 +470,13 @@ __global__ __launch_bounds__(256) void attention_bf16_kernel(AttnArgs p) {
     // Scale, mask (only blocks that cross some query's visible range), online
     // softmax; the output is rescaled only when some query's reference max
     // moved, and never on the first block (the output is still zero).
-    const bool masked = !text_mask && __any(key0 < klo || key0 + kAttnKV - 1 > khi);
+    const bool masked = !text_mask && __any(key0 < klo || key0 + KV - 1 > khi);
     bool rescale;
     if (p.rel_bias) attn_rel_bias(p, sc, h, qi, key0, fg);
-    const float alpha = attn_softmax_block(sc, key0, fg, klo, khi, masked,
-                                           p.rel_bias ? 1.44269504088896341f : cs, mrun,
-                                           lrun, rescale);
+    constexpr int kSlack = T == 2 && KV == 32 ? 1 : 8;
+    const float alpha = attn_softmax_block<NT, kSlack>(sc, key0, fg, klo, khi, masked,
+                                                       p.rel_bias ? 1.44269504088896341f : cs,
+                                                       mrun, lrun, rescale);
     if (rescale && kb != kb_lo) {
 #pragma unroll
       for (int t = 0; t < DT; t++)
@@ -629,10 +484,10 @@ __global__ __launch_bounds__(256) void attention_bf16_kernel(AttnArgs p) {
         for (int e = 0; e < 16; e++) o[t][e] *= alpha;
     }
 
-    // O^T += V^T · P^T over 4 chunks of 16 keys; lane half g, element e of
+    // O^T += V^T · P^T over chunks of 16 keys; lane half g, element e of
     // chunk kc is register sc[kc/2][(kc%2)*8 + e], key 16kc + 8(e/4) + 4g + e%4.
 #pragma unroll
-    for (int kc = 0; kc < 4; kc++) {
+    for (int kc = 0; kc < 2 * NT; kc++) {
       v8bf ph, pl;
       if constexpr (T == 2) {
         attn_split8(sc[kc >> 1], (kc & 1) * 8, ph, pl);
@@ -654,7 +509,9 @@ __global__ __launch_bounds__(256) void attention_bf16_kernel(AttnArgs p) {
     }
     }
 
-    __syncthreads();  // next block landed (vmcnt) and this block's reads are done
+    if constexpr (F32)
+      if (next) stash(kb + 1, buf ^ 1);
+    __syncthreads();  // next block landed and this block's reads are done
   }
 
   const float ltot = lrun + __shfl_xor(lrun, 32, 64);
@@ -889,17 +746,23 @@ __global__ __launch_bounds__(64 * kH256Waves) void attention_h256_kernel(AttnArg
   }
 }
 
+// Three-term products: keys per LDS block and waves per SIMD. 32 keys of head
+// dim 32 are too few for a DMA instruction per wave; planes of head dim 64 gain
+// 4 % alone and nothing inside a full-int8 forward, so they keep 64 keys (and
+// with them the bits that its quantizers see).
+template <int DH, bool F32>
+constexpr int kKV3 = DH >= (F32 ? 64 : 128) ? 32 : kAttnKV;
+template <int DH>
+constexpr int kMinW3 = DH == 256 ? 1 : 2;
+
 template <int DH>
 static hipError_t launch_attn_dh(const AttnArgs& a, int precision, hipStream_t s) {
   const int units = a.batch * a.kv_heads;
   const dim3 grid(8 * ceil_div(a.max_len, kAttnQ) * (a.heads / a.kv_heads) * ceil_div(units, 8));
-  if (a.in_bf16 == 2) {  // hi/lo planes: the three-term products, pipelined
-    if constexpr (DH <= 128) {
-      if (precision != 3 || !a.qkv_lo) return hipErrorInvalidValue;
-      timed_launch((attention_bf16_kernel<DH, 2>), grid, dim3(256), 0, s, a);
-    } else {
-      return hipErrorInvalidValue;
-    }
+  if (a.in_bf16 == 2) {  // hi/lo planes: the three-term products
+    if (precision != 3 || !a.qkv_lo) return hipErrorInvalidValue;
+    timed_launch((attention_bf16_kernel<DH, 2, kKV3<DH, false>, false, kMinW3<DH>>), grid, dim3(256),
+                 0, s, a);
   } else if (a.in_bf16) {  // bf16 input carries no low half: one-term products
     // head dim 256: the 16x16x32 kernel (two waves per SIMD; 324 against 372
     // µs at EmbeddingGemma's global layer, 186 against 219 at its window-512
@@ -907,12 +770,13 @@ static hipError_t launch_attn_dh(const AttnArgs& a, int precision, hipStream_t s
     if (DH == 256 && !a.rel_bias)
       timed_launch(attention_h256_kernel, grid, dim3(64 * kH256Waves), 0, s, a);
     else
-      timed_launch((attention_bf16_kernel<DH, 1>), grid, dim3(256), 0, s, a);
+      timed_launch((attention_bf16_kernel<DH, 1, kAttnKV, false, 1>), grid, dim3(256), 0, s, a);
   }
   else if (precision == 3)
-    timed_launch((attention_kernel<DH, 3, float>), grid, dim3(256), 0, s, a);
+    timed_launch((attention_bf16_kernel<DH, 2, kKV3<DH, true>, true, kMinW3<DH>>), grid, dim3(256),
+                 0, s, a);
   else
-    timed_launch((attention_kernel<DH, 1, float>), grid, dim3(256), 0, s, a);
+    timed_launch((attention_bf16_kernel<DH, 1, kAttnKV, true, 1>), grid, dim3(256), 0, s, a);
   return hipGetLastError();
 }
 

@@ -214,7 +214,9 @@ hipError_t launch_rms_residual(const RmsArgs& a, hipStream_t s) {
 // row's position (applyRoPE, modernbert.go:130-143: each product rounded to
 // float32 before the add). With `outh` the results
 // go to bf16 rows of the same layout instead (round to nearest even), and
-// the v heads are converted too: the operands of a bf16 attention.
+// the v heads are converted too: the operands of a bf16 attention. With
+// `outl` as well, outh and outl receive the bf16 hi/lo split of the results,
+// the operands of an fp32-grade attention.
 // A wave takes kQkItems consecutive items, loading all of them before it
 // reduces, so their memory latencies overlap.
 constexpr int kQkItems = 4;
@@ -223,7 +225,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(
     float* __restrict__ qkv, int ldqkv, int m, int nq, int nkv, int dh,
     const float* __restrict__ q_g, const float* __restrict__ k_g, float eps,
     const float* __restrict__ cos_t, const float* __restrict__ sin_t,
-    const int32_t* __restrict__ pos, __bf16* __restrict__ outh) {
+    const int32_t* __restrict__ pos, __bf16* __restrict__ outh, __bf16* __restrict__ outl) {
   const int lane = threadIdx.x & 63;
   const int item0 = (blockIdx.x * kRows + (threadIdx.x >> 6)) * kQkItems;
   const int nh = nq + nkv + (outh ? nkv : 0);
@@ -249,13 +251,20 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(
     const int row = item / nh, h = item % nh;
     float* v = qkv + (size_t)row * ldqkv + h * dh;
     __bf16* o = outh ? outh + (size_t)row * ldqkv + h * dh : nullptr;
+    __bf16* ol = outl ? outl + (size_t)row * ldqkv + h * dh : nullptr;
+    auto store = [&](int d, float x) {
+      __bf16 hi, lo;
+      split_hi_lo(x, hi, lo);
+      o[d] = hi;
+      if (ol) ol[d] = lo;
+    };
     if (h >= nq + nkv) {  // v head: conversion only
 #pragma unroll
       for (int e = 0; e < 2; e++) {
         const int d = lane + 64 * e;
         if (d < half) {
-          o[d] = (__bf16)x1[it][e];
-          o[d + half] = (__bf16)x2[it][e];
+          store(d, x1[it][e]);
+          store(d + half, x2[it][e]);
         }
       }
       continue;
@@ -277,8 +286,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(
         const float cc = c[d], ssn = sn[d];
         const float t0 = a * cc, t1 = b * ssn, t2 = b * cc, t3 = a * ssn;
         if (o) {
-          o[d] = (__bf16)(t0 - t1);
-          o[d + half] = (__bf16)(t2 + t3);
+          store(d, t0 - t1);
+          store(d + half, t2 + t3);
         } else {
           v[d] = t0 - t1;
           v[d + half] = t2 + t3;
@@ -299,8 +308,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_vec_kernel(
     float* __restrict__ qkv, int ldqkv, int nq, int nkv, const float* __restrict__ q_g,
     const float* __restrict__ k_g, float eps, const float* __restrict__ cos_t,
     const float* __restrict__ sin_t, const int32_t* __restrict__ pos,
-    __bf16* __restrict__ outh) {
-  typedef __bf16 v4bf __attribute__((ext_vector_type(4)));
+    __bf16* __restrict__ outh, __bf16* __restrict__ outl) {
   constexpr int LPH = DH / 4;    // lanes per head
   constexpr int HPW = 64 / LPH;  // heads per wave
   constexpr int HALF = DH / 2;
@@ -331,8 +339,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_vec_kernel(
       for (int o = LPH / 2; o >= 1; o >>= 1) ss += __shfl_xor(ss, o, 64);
       if (h >= nh) continue;
       if (h >= nq + nkv) {  // v head: conversion only
-        *reinterpret_cast<v4bf*>(outh + off) =
-            v4bf{(__bf16)x[it][0], (__bf16)x[it][1], (__bf16)x[it][2], (__bf16)x[it][3]};
+        store_planes4(outh, outl, off, x[it]);
         continue;
       }
       const float inv = rms_inv(ss, DH, eps);
@@ -358,8 +365,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_vec_kernel(
         o[c] = first ? a * cc[c] - b * sn[c] : b * cc[c] + a * sn[c];
       }
       if (outh)
-        *reinterpret_cast<v4bf*>(outh + off) =
-            v4bf{(__bf16)o[0], (__bf16)o[1], (__bf16)o[2], (__bf16)o[3]};
+        store_planes4(outh, outl, off, o);
       else
         *reinterpret_cast<v4f*>(qkv + off) = o;
     }
@@ -369,26 +375,27 @@ __global__ __launch_bounds__(256) void qk_norm_rope_vec_kernel(
 hipError_t launch_qk_norm_rope(float* qkv, int ldqkv, int m, int nq, int nkv, int dh,
                                const float* q_g, const float* k_g, float eps,
                                const float* cos_t, const float* sin_t,
-                               const int32_t* pos, __bf16* outh, hipStream_t s) {
+                               const int32_t* pos, __bf16* outh, __bf16* outl, hipStream_t s) {
   if (m <= 0) return hipSuccess;
-  if (dh % 2 || dh > 256) return hipErrorInvalidValue;
+  if (dh % 2 || dh > 256 || (outl && !outh)) return hipErrorInvalidValue;
   const bool vec = ldqkv % 4 == 0 && ((reinterpret_cast<uintptr_t>(qkv) & 15) == 0) &&
-                   ((reinterpret_cast<uintptr_t>(outh) & 7) == 0);
+                   ((reinterpret_cast<uintptr_t>(outh) & 7) == 0) &&
+                   ((reinterpret_cast<uintptr_t>(outl) & 7) == 0);
   if (vec && (dh == 64 || dh == 128 || dh == 256)) {
     if (dh == 64)
       hipLaunchKernelGGL((qk_norm_rope_vec_kernel<64>), dim3(m), dim3(256), 0, s, qkv, ldqkv, nq,
-                         nkv, q_g, k_g, eps, cos_t, sin_t, pos, outh);
+                         nkv, q_g, k_g, eps, cos_t, sin_t, pos, outh, outl);
     else if (dh == 128)
       hipLaunchKernelGGL((qk_norm_rope_vec_kernel<128>), dim3(m), dim3(256), 0, s, qkv, ldqkv,
-                         nq, nkv, q_g, k_g, eps, cos_t, sin_t, pos, outh);
+                         nq, nkv, q_g, k_g, eps, cos_t, sin_t, pos, outh, outl);
     else
       hipLaunchKernelGGL((qk_norm_rope_vec_kernel<256>), dim3(m), dim3(256), 0, s, qkv, ldqkv,
-                         nq, nkv, q_g, k_g, eps, cos_t, sin_t, pos, outh);
+                         nq, nkv, q_g, k_g, eps, cos_t, sin_t, pos, outh, outl);
     return hipGetLastError();
   }
   const int items = m * (nq + nkv + (outh ? nkv : 0));
   hipLaunchKernelGGL(qk_norm_rope_kernel, dim3(ceil_div(items, kRows * kQkItems)), dim3(256), 0,
-                     s, qkv, ldqkv, m, nq, nkv, dh, q_g, k_g, eps, cos_t, sin_t, pos, outh);
+                     s, qkv, ldqkv, m, nq, nkv, dh, q_g, k_g, eps, cos_t, sin_t, pos, outh, outl);
   return hipGetLastError();
 }
 

@@ -173,7 +173,8 @@ struct rh_model {
   size_t cap_ids = 0;
   float *x = nullptr, *qkv = nullptr, *ctxb = nullptr, *y = nullptr, *hid = nullptr;
   float* hid2 = nullptr;  // [cap][I] up rows of a layer whose gate and up are separate
-  __bf16* qkvh = nullptr;                 // bf16 QKV rows (bf16 attention)
+  __bf16* qkvh = nullptr;                 // bf16 QKV rows (bf16 attention), or their hi plane
+  __bf16* qkvl = nullptr;                 // RoPE family, fp32-grade attention: the lo plane
   // bf16 hi/lo activation planes written by the producers of the
   // weight-only int8 / fp32 GEMMs: p0 [cap][ld0] holds a width-H or
   // width-qdim input (normed rows, attention output), p1 [cap][ld1] the
@@ -217,7 +218,7 @@ struct rh_model {
 
   void release_ws() {
     for (void* p : {(void*)x, (void*)qkv, (void*)ctxb, (void*)y, (void*)hid, (void*)qa,
-                    (void*)rs, (void*)cu_d, (void*)ids_d, (void*)out_d, (void*)qkvh,
+                    (void*)rs, (void*)cu_d, (void*)ids_d, (void*)out_d, (void*)qkvh, (void*)qkvl,
                     (void*)qa2, (void*)rs2, (void*)absmax, (void*)normed, (void*)pooled,
                     (void*)dense_hid, (void*)p0h, (void*)p0l, (void*)p1h, (void*)p1l,
                     (void*)pos_d, (void*)hid2, (void*)qslots, (void*)qsync})
@@ -227,7 +228,7 @@ struct rh_model {
     hid2 = nullptr;
     pos_d = nullptr;
     qa = qa2 = nullptr;
-    qkvh = p0h = p0l = p1h = p1l = nullptr;
+    qkvh = qkvl = p0h = p0l = p1h = p1l = nullptr;
     cu_d = ids_d = nullptr;
     cap = cap_batch = cap_ids = 0;
   }
@@ -342,14 +343,14 @@ struct rh_model {
     if (rows > cap) {
       int newcap = (int)round_up(rows, 256);
       for (void* p : {(void*)x, (void*)qkv, (void*)ctxb, (void*)y, (void*)hid, (void*)qa,
-                      (void*)rs, (void*)qkvh, (void*)qa2, (void*)rs2, (void*)absmax,
+                      (void*)rs, (void*)qkvh, (void*)qkvl, (void*)qa2, (void*)rs2, (void*)absmax,
                       (void*)normed, (void*)pos_d, (void*)p0h, (void*)p0l, (void*)p1h,
                       (void*)p1l, (void*)hid2, (void*)qslots, (void*)qsync})
         if (p) RH_HIP(hipFree(p));
       x = qkv = ctxb = y = hid = rs = rs2 = absmax = normed = hid2 = nullptr;
       qslots = qsync = nullptr;
       qa = qa2 = nullptr;
-      qkvh = p0h = p0l = p1h = p1l = nullptr;
+      qkvh = qkvl = p0h = p0l = p1h = p1l = nullptr;
       pos_d = nullptr;
       const size_t r = newcap;
       RH_HIP(dalloc(&x, r * H));
@@ -383,6 +384,9 @@ struct rh_model {
       }
       cap = newcap;
     }
+    // q|k|v's lo plane, for the models that attend at fp32 grade
+    if (rope_family() && attn_precision == 3 && !qkvl)
+      RH_HIP(dalloc(&qkvl, (size_t)cap * qkv_width()));
     if (batch > cap_batch) {
       if (cu_d) RH_HIP(hipFree(cu_d));
       if (out_d) RH_HIP(hipFree(out_d));
@@ -1021,6 +1025,8 @@ int rh_model::forward_dec(const int32_t* ids_dev, int stride, const std::vector<
     const bool local = (gemma() || modernbert()) && !L.global;
     // bf16 attention reads bf16 q|k|v rows: written by the q|k|v GEMM's
     // QK-norm + RoPE epilogue where that applies, else by the separate pass
+    // (and fp32-grade attention their hi/lo planes, which that pass splits once
+    // where attention would for every block of queries)
     const bool hb = attn_precision == 1;
     bool fused_qk = false;
     if (qk_epilogue && hb && L.qkv && L.q_norm && planes_in(L.qkv)) {
@@ -1047,11 +1053,12 @@ int rh_model::forward_dec(const int32_t* ids_dev, int stride, const std::vector<
     if (!fused_qk) {
       RH_HIP(launch_qk_norm_rope(qkvp, qkvw, Mp, nq(), nkv(), dh(), L.q_norm, L.k_norm, e,
                                  local ? cos_l : cos_g, local ? sin_l : sin_g, pos_d + r0,
-                                 hb ? qkvh + r0 * qkvw : nullptr, ps));
+                                 qkvh + r0 * qkvw, hb ? nullptr : qkvl + r0 * qkvw, ps));
     }
     AttnArgs aa{};
-    aa.qkv = hb ? (const void*)qkvh : (const void*)qkv;  // rows are absolute (cu)
-    aa.in_bf16 = hb ? 1 : 0;
+    aa.qkv = qkvh;  // rows are absolute (cu)
+    aa.qkv_lo = hb ? nullptr : qkvl;
+    aa.in_bf16 = hb ? 1 : 2;
     aa.ldqkv = qkvw;
     aa.q_off = 0;
     aa.k_off = qd;

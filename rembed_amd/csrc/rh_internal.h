@@ -386,8 +386,8 @@ struct AttnArgs {
   int rel_center;
 };
 // precision: 1 = bf16 MFMA, 3 = three-term bf16 split (fp32-grade; with
-// in_bf16 2 the split arrives as hi/lo planes and runs on the pipelined
-// kernel, dh <= 128)
+// in_bf16 2 the split arrives as hi/lo planes, else the kernel splits the
+// fp32 rows)
 hipError_t launch_attention(const AttnArgs& a, int precision, hipStream_t s);
 // The same attention in the reference's float32 operation order
 // (MatMulSerial/dot4, Softmax; attention_exact.hip): bit-identical context
@@ -432,7 +432,7 @@ hipError_t launch_rms_residual(const RmsArgs& a, hipStream_t s);
 hipError_t launch_qk_norm_rope(float* qkv, int ldqkv, int m, int nq, int nkv, int dh,
                                const float* q_g, const float* k_g, float eps,
                                const float* cos_t, const float* sin_t,
-                               const int32_t* pos, __bf16* outh, hipStream_t s);
+                               const int32_t* pos, __bf16* outh, __bf16* outl, hipStream_t s);
 // EmbeddingGemma Dense head (gemma3.go:174-198) on pooled [batch][H] rows:
 // out = W2 . (W1 . pooled), float32 sequential sums; optional L2. The
 // weights are given transposed: w1T [H][D], w2T [D][H]; hid is [batch][D].

@@ -152,6 +152,45 @@ def test_attention_kernels(gpu_ctx, case):
         assert err_p <= 1e-4 * (1 + np.abs(want_f).max())
 
 
+@pytest.mark.parametrize("dh", [32, 64, 128, 256])
+@pytest.mark.parametrize("causal,window", [(False, 0), (True, 0), (False, 33), (True, 70)])
+def test_fp32_rows_at_key_block_edges(gpu_ctx, dh, causal, window):
+    """fp32 rows at fp32-grade precision, texts that end at, before and after
+    the 32- and 64-key blocks and the 128-query workgroups. At head dims 32 and
+    128, whose blocks are of one size, the planes of the same split give the same
+    bits (the products and their order are the same, only the staging differs)."""
+    heads, kv_heads = 4, 2
+    lens = [1, 31, 32, 33, 63, 64, 65, 96, 97, 128, 129, 161]
+    say(f"fp32 rows dh={dh} causal={causal} window={window}")
+    rng = np.random.default_rng(dh + causal + window)
+    M, ld = sum(lens), (heads + 2 * kv_heads) * dh
+    q_off, k_off, v_off = 0, heads * dh, (heads + kv_heads) * dh
+    x = rng.standard_normal((M, ld)).astype(np.float32)
+    scale = 1.0 / np.sqrt(dh)
+    cu = gpu_ctx.upload(np.concatenate([[0], np.cumsum(lens)]).astype(np.int32))
+
+    def run(call, *buf):
+        out = gpu_ctx.upload(np.full((M, heads * dh), np.nan, np.float32))
+        call(gpu_ctx, out, heads * dh, *buf, ld, q_off, k_off, v_off, cu, len(lens), max(lens),
+             heads, kv_heads, dh, scale, causal, window, *((3,) if call is T.Attention else ()))
+        gpu_ctx.sync()
+        return out.download(np.float32, (M, heads * dh))
+
+    got = run(T.Attention, gpu_ctx.upload(x), 0)
+    want = reference(x, lens, heads, kv_heads, dh, scale, causal, window, q_off, k_off, v_off)
+    # operands are split to 2^-17 of a value (and lo·lo, below 2^-18, is left
+    # out): a score is off by at most 3·2^-17 · scale · |q||k|, a weight by that
+    # relative to itself (twice: its own score's and the sum's) plus its split
+    qk = scale * np.linalg.norm(x[:, :k_off].reshape(-1, dh), axis=1).max() * \
+        np.linalg.norm(x[:, k_off:v_off].reshape(-1, dh), axis=1).max()
+    bound = (2 * 3 * qk + 6) * 2.0 ** -17 * np.abs(x[:, v_off:]).max()
+    assert np.abs(got - want).max() <= bound
+    if dh in (32, 128):
+        hi = to_bf16_bits(x)
+        lo = to_bf16_bits(x - bf16_value(hi))
+        assert np.array_equal(run(T.AttentionPlanes, gpu_ctx.upload(hi), gpu_ctx.upload(lo)), got)
+
+
 def test_attention_argument_errors(gpu_ctx):
     from rembed_amd._lib import RembedError
     buf = gpu_ctx.alloc(4096)
