@@ -170,11 +170,12 @@ def test_row_kernels_few_and_many_rows_agree(gpu_ctx, n):
     for k in (1, 2048, m):
         dx = gpu_ctx.upload(x[:k])
         _lib.check(_lib.lib.rh_layernorm(gpu_ctx.h, dx.ptr, g.ptr, b.ptr, k, n, 1e-12))
-        da, dq, ds = gpu_ctx.upload(x[:k]), gpu_ctx.alloc(k * n), gpu_ctx.alloc(k * 4)
-        T.QuantizeRowsU8(gpu_ctx, da, k, n, dq, n, ds)
+        ldq = T.ldq_for(n)
+        da, dq, ds = gpu_ctx.upload(x[:k]), gpu_ctx.alloc(k * ldq), gpu_ctx.alloc(k * 4)
+        T.QuantizeRowsU8(gpu_ctx, da, k, n, dq, ldq, ds)
         gpu_ctx.sync()
         ln[k] = dx.download(np.float32, (k, n))
-        qs[k] = dq.download(np.uint8, (k, n))
+        qs[k] = dq.download(np.uint8, (k, ldq))[:, :n]
     assert np.array_equal(ln[2048][:1], ln[1]) and np.array_equal(ln[m][:2048], ln[2048])
     assert np.array_equal(qs[2048][:1], qs[1]) and np.array_equal(qs[m][:2048], qs[2048])
     assert np.array_equal(qs[m], np.stack([O.quantize_row_u8(r)[0] for r in x]))
