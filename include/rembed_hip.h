@@ -74,13 +74,10 @@ void *rh_context_stream(rh_context *ctx);
  *   RH_CTX_BF_ALGO   weight-only int8 / fp32 GEMMs: 0 = activations split
  *                    once into bf16 hi/lo planes and weights stored as bf16
  *                    planes (default), 1 = split inside the GEMM's main loop
- *   RH_CTX_BF_TILE   tile of the bf16-planes GEMM: 0 = automatic, 1 = 256x256,
- *                    2 = 256x128, 3 = 128x128, 4 = 256x256, 5 = 256x128
- *                    (eight waves), 6 = 256x256, 7 = 256x128 (eight waves,
- *                    128-byte k stages), 8 = 64x64, 9 = 128x64 (four waves),
- *                    10 = 128x256 (eight waves, three 64-byte k stages, two
- *                    workgroups per CU); 6, 7 and 10 for the one-term
- *                    weight-only int8 product only, the other products take 3
+ *   RH_CTX_BF_TILE   tile of the bf16-planes GEMM: 0 = automatic, 1, 4 and 6 =
+ *                    256x256, 2, 5 and 7 = 256x128, 3 = 128x128, 8 = 64x64,
+ *                    9 = 128x64, 10 = 128x256 (one-term weight-only int8
+ *                    product; the other products take 3)
  *   RH_CTX_TILE_GROUP  GEMM tile order: consecutive workgroups walk this many
  *                    row blocks down a column block (1 = row-major; default 4) */
 #define RH_CTX_F32_ALGO 1

@@ -476,7 +476,7 @@ int run_linear_qk(Context* ctx, const rh_weight* w, const Planes& pin, int m,
     return RH_OK;
   if (w->n % 256 != 0 || !(q.dh == 64 || q.dh == 128 || q.dh == 256) || ldo % 4 != 0)
     return RH_OK;
-  // the fused tile only where the 256x256 grid keeps the CUs busy, and
+  // the fused form only where 256x256 tiles would keep half the CUs busy, and
   // without row chunking (32-bit element offsets)
   if ((long long)ceil_div(m, 256) * (w->n / 256) < 128) return RH_OK;
   if ((long long)m * std::max(pin.ld, ldo) >= (1LL << 30)) return RH_OK;

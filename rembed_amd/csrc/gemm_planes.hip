@@ -15,13 +15,20 @@
 //    lo·lo term is ~2^-16 of the others, below the fp32 rounding of the sum
 //    at these magnitudes).
 //
-// Main loop (same scheme as the int8 GEMM): BM x BN tile per 256-thread
-// workgroup, 2x2 waves of 32x32 MFMA tiles, K in stages of 32 bf16 = 64
-// bytes per row and plane. Stages reach LDS by global_load_lds_dwordx4 (no
-// register staging): lane l of a wave instruction writes LDS bytes
-// [16l, 16l+16) of a 1 KiB block, so each lane loads the global 16-byte chunk
-// that belongs at that slot, rows permuted by i8_slot (conflict-free fragment
-// reads). NS stages in flight, one barrier per stage.
+// Main loop: BM x BN tile per workgroup, a WGM x WGN grid of waves of 32x32
+// MFMA tiles, K in stages of BK bf16 per row and plane. Stages reach LDS by
+// global_load_lds_dwordx4 (no register staging): lane l of a wave instruction
+// writes LDS bytes [16l, 16l+16) of a 1 KiB block, so each lane loads the
+// global 16-byte chunk that belongs at that slot, rows permuted for
+// conflict-free fragment reads. NS stages in flight, one barrier per stage; a
+// step's fragments are read from LDS under the products of the step before.
+//
+// What bounds it: what one CU pulls. Probes of global_load_lds on MI355X, one
+// workgroup per CU and L2 hits, B/ns per CU: 16 rows of 64 bytes per
+// instruction 53 with four waves and 69-72 with eight, 8 rows of 128 bytes
+// 59 and 84-89. Hence 128-byte rows (BK 64) and eight waves on a CU: one
+// 512-thread workgroup, two 64-KiB ones, or four multiplying waves and LW more
+// that only load.
 //
 // The epilogue parks each 32-row band of accumulators in LDS and reads rows
 // back 4 columns per lane: scale, bias, activation (or the gated pair) and a
@@ -30,20 +37,31 @@
 
 namespace rh {
 
-// WGN waves along N (2: a 2x2 grid of 4 waves; 4: a 2x4 grid of 8 waves, two
-// per SIMD, so one wave's LDS waits overlap the other's MFMAs).
-// BK: k elements per stage and row, 32 (64-byte rows, i8_slot permutation)
-// or 64 (128-byte rows, lds_off permutation; half the barriers).
+// Wait until this wave's loads of at most min(MAX, later) stages are pending.
+template <int LOADS, int MAX>
+__device__ __forceinline__ void wait_stages(int later) {
+  if constexpr (MAX == 0) {
+    wait_vmcnt<0>();
+  } else {
+    if (later >= MAX) wait_vmcnt<MAX * LOADS>();
+    else wait_stages<LOADS, MAX - 1>(later);
+  }
+}
+
+// WGM x WGN waves multiply, LW more only load. BK: k elements per stage and
+// row, 32 (64-byte rows, i8_slot permutation) or 64 (128-byte rows, lds_off
+// permutation; half the barriers).
 // QKN: the QK-norm + RoPE epilogue of the decoders' q|k|v projection (bf16
 // rows to p.qk_out; see GemmPlArgs).
-template <int BM, int BN, int NS, int AT, int BT, bool GLU, int WGN = 2, int BK = 32,
+template <int BM, int BN, int NS, int AT, int BT, bool GLU, int BK, int WGM, int WGN, int LW = 0,
           bool QKN = false>
-__global__ __launch_bounds__(128 * WGN) void gemm_planes_kernel(GemmPlArgs p) {
-  constexpr int NT = 128 * WGN;  // threads
-  constexpr int NW = 2 * WGN;    // waves
+__global__ __launch_bounds__(64 * (WGM * WGN + LW),
+                             QKN ? 4 : 1) void gemm_planes_kernel(GemmPlArgs p) {
+  constexpr int NW = WGM * WGN;        // waves that multiply
+  constexpr int NT = 64 * (NW + LW);   // threads
   constexpr int CPR = BK / 8;    // 16-byte chunks per row
   static_assert(BK == 32 || BK == 64, "stage depth");
-  constexpr int WM = BM / 2, WN = BN / WGN;
+  constexpr int WM = BM / WGM, WN = BN / WGN;
   constexpr int TM = WM / 32, TN = WN / 32;
   constexpr int kA = BM * BK * 2, kB = BN * BK * 2;  // bytes per plane
   constexpr int kStage = AT * kA + BT * kB;
@@ -52,12 +70,13 @@ __global__ __launch_bounds__(128 * WGN) void gemm_planes_kernel(GemmPlArgs p) {
   constexpr int kEpiStride = WN + 4;  // floats per row of the epilogue transpose
   static_assert(LA >= 1 && LB >= 1 && TN >= 1, "tile too small for the wave grid");
   // A stage's slot is refilled right after the barrier that follows the
-  // last reads of it, so two slots suffice (one stage in flight).
+  // last reads of it, so two slots suffice.
   static_assert(NS >= 2, "ring");
-  static_assert(NS * kStage <= 160 * 1024, "LDS");
-  static_assert(NS * kStage >= NW * 32 * kEpiStride * 4, "epilogue LDS");
-  static_assert((NS - 2) * kLoads < 64, "vmcnt range");
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[NS * kStage];
+  constexpr int kEpi = NW * 32 * kEpiStride * 4;  // epilogue bands
+  constexpr int kLds = NS * kStage > kEpi ? NS * kStage : kEpi;
+  static_assert(kLds <= 160 * 1024, "LDS");
+  static_assert((NS - 1) * kLoads < 64, "vmcnt range");
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[kLds];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -116,51 +135,80 @@ __global__ __launch_bounds__(128 * WGN) void gemm_planes_kernel(GemmPlArgs p) {
 #pragma unroll
       for (int e = 0; e < 16; e++) acc[i][j][e] = 0.0f;
 
-#pragma unroll
-  for (int st = 0; st < NS - 1; st++)
-    if (st < nk) issue(st);
-
   const int fr = lane & 31, fg = lane >> 5;
-  for (int kt = 0; kt < nk; kt++) {
-    // Stage kt has landed once at most min(NS-2, nk-1-kt) later stages are
-    // still pending for this wave.
-    const int later = nk - 1 - kt;
-    if (later >= NS - 2) wait_vmcnt<(NS - 2) * kLoads>();
-    else if (NS > 3 && later == 1) wait_vmcnt<kLoads>();
-    else wait_vmcnt<0>();
-    // A bare s_barrier (a __syncthreads() fence would drain the whole ring):
-    // every wave's stage-kt data is in LDS and its reads of stage kt-1 are
-    // done, so the slot of stage kt-1 can be refilled.
-    __builtin_amdgcn_s_barrier();
-    if (kt + NS - 1 < nk) issue(kt + NS - 1);
+  // The fragments of one 16-k step, held twice: step s + 1 (the next stage's
+  // first, past the barrier, after a stage's last) is read from LDS under the
+  // products of step s.
+  struct Frags {
+    v8bf a[AT][TM], b[BT][TN];
+  };
+  auto read = [&](Frags& f, int kt, int s) {
     const uint8_t* sA = lds + (kt % NS) * kStage;
     const uint8_t* sB = sA + AT * kA;
+    const int c = 2 * s + fg;
 #pragma unroll
-    for (int s = 0; s < BK / 16; s++) {
-      const int c = 2 * s + fg;
-      v8bf fah[TM], fal[TM], fbh[TN], fbl[TN];
+    for (int i = 0; i < TM; i++) {
+      const int off = stage_frag_off<BK * 2>(wm * WM + i * 32 + fr, c);
 #pragma unroll
-      for (int i = 0; i < TM; i++) {
-        const int off = stage_frag_off<BK * 2>(wm * WM + i * 32 + fr, c);
-        fah[i] = *reinterpret_cast<const v8bf*>(sA + off);
-        if constexpr (AT == 2) fal[i] = *reinterpret_cast<const v8bf*>(sA + kA + off);
-      }
+      for (int x = 0; x < AT; x++) f.a[x][i] = *reinterpret_cast<const v8bf*>(sA + x * kA + off);
+    }
 #pragma unroll
-      for (int j = 0; j < TN; j++) {
-        const int off = stage_frag_off<BK * 2>(wn * WN + j * 32 + fr, c);
-        fbh[j] = *reinterpret_cast<const v8bf*>(sB + off);
-        if constexpr (BT == 2) fbl[j] = *reinterpret_cast<const v8bf*>(sB + kB + off);
-      }
+    for (int j = 0; j < TN; j++) {
+      const int off = stage_frag_off<BK * 2>(wn * WN + j * 32 + fr, c);
+#pragma unroll
+      for (int x = 0; x < BT; x++) f.b[x][j] = *reinterpret_cast<const v8bf*>(sB + x * kB + off);
+    }
+  };
+  // hi·hi, then hi·lo, then lo·hi of every tile: an output's sums keep their
+  // order and no product waits for the one before it
+  auto multiply = [&](const Frags& f) {
+#pragma unroll
+    for (int x = 0; x < AT + BT - 1; x++)
 #pragma unroll
       for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int j = 0; j < TN; j++) {
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fah[i], fbh[j], acc[i][j], 0, 0, 0);
-          if constexpr (BT == 2)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fah[i], fbl[j], acc[i][j], 0, 0, 0);
-          if constexpr (AT == 2)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fal[i], fbh[j], acc[i][j], 0, 0, 0);
+        for (int j = 0; j < TN; j++)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              f.a[x == BT ? 1 : 0][i], f.b[x == 1 && BT == 2 ? 1 : 0][j], acc[i][j], 0, 0, 0);
+  };
+
+#pragma unroll
+  for (int st = 0; st < NS; st++)
+    if (st < nk) issue(st);
+  wait_stages<kLoads, NS - 1>(nk - 1);  // stage 0 has landed for this wave
+  stage_barrier();                      // and for the others
+  // To stage kt + 1: this wave's loads of it have landed once only those of the
+  // later stages issued are pending. Past the barrier that holds for every wave
+  // (a __syncthreads() fence would drain the ring) and all reads of stage kt are
+  // done, so its slot can be refilled.
+  auto advance = [&](int kt) {
+    wait_stages<kLoads, NS - 2>(nk - 2 - kt);
+    stage_barrier();
+    if (kt + NS < nk) issue(kt + NS);
+  };
+  if (LW > 0 && wave >= NW) {
+    for (int kt = 0; kt + 1 < nk; kt++) advance(kt);
+  } else {
+    constexpr int S = BK / 16;
+    Frags f[2];
+    read(f[0], 0, 0);
+    for (int kt = 0; kt + 1 < nk; kt++) {
+#pragma unroll
+      for (int s = 0; s < S; s++) {
+        if (s + 1 < S) {
+          read(f[(s + 1) & 1], kt, s + 1);
+        } else {
+          wait_lgkmcnt0();
+          advance(kt);
+          read(f[0], kt + 1, 0);
         }
+        multiply(f[s & 1]);
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < S; s++) {
+      if (s + 1 < S) read(f[(s + 1) & 1], nk - 1, s + 1);
+      multiply(f[s & 1]);
     }
   }
 
@@ -168,20 +216,19 @@ __global__ __launch_bounds__(128 * WGN) void gemm_planes_kernel(GemmPlArgs p) {
   // applyDense order (bert.go:282-301, pack8.go:118-122): fp32 sum, ·scale
   // (weight-only int8), + bias, then the activation.
   __syncthreads();
+  if (LW > 0 && wave >= NW) return;
   float* ep = reinterpret_cast<float*>(lds) + wave * 32 * kEpiStride;
   // QKN: this lane's column scales, bias and norm weights (fixed columns
   // 4*lane..+3 of the tile for every row)
   v4f qk_cs = {1.0f, 1.0f, 1.0f, 1.0f}, qk_bs = {0.0f, 0.0f, 0.0f, 0.0f};
   v4f qk_g = {1.0f, 1.0f, 1.0f, 1.0f};
-  // and the positions of this wave row's WM rows (lane r: rows r, 64 + r),
-  // read per row with readlane: no dependent global load before a row's
-  // cos/sin loads
-  int qk_pos0 = 0, qk_pos1 = 0;
+  // and the positions of this wave row's WM rows (lane r: row r), read per row
+  // with readlane: no dependent global load before a row's cos/sin loads
+  int qk_pos0 = 0;
   if constexpr (QKN) {
-    static_assert(WM == 128, "two position registers cover the wave row");
+    static_assert(WM <= 64, "one position register covers the wave row");
     const int r = row0 + wm * WM + lane;
     qk_pos0 = r < p.M ? p.qk_pos[r] : 0;
-    qk_pos1 = r + 64 < p.M ? p.qk_pos[r + 64] : 0;
     const int gcol = col0 + lane * 4, h = gcol / p.qk_dh, d = gcol % p.qk_dh;
     if (p.col_scales) qk_cs = *reinterpret_cast<const v4f*>(p.col_scales + gcol);
     if (p.bias) qk_bs = *reinterpret_cast<const v4f*>(p.bias + gcol);
@@ -225,7 +272,7 @@ __global__ __launch_bounds__(128 * WGN) void gemm_planes_kernel(GemmPlArgs p) {
 #pragma unroll
       for (int k = 0; k < RPW; k++) {
         const int wr = i * 32 + wn + k * WGN;  // row within the wave row (uniform)
-        const int pos = __builtin_amdgcn_readlane(wr < 64 ? qk_pos0 : qk_pos1, wr & 63);
+        const int pos = __builtin_amdgcn_readlane(qk_pos0, wr);
         ccs[k] = *reinterpret_cast<const v4f*>(p.qk_cos + (size_t)pos * half + dp);
         sns[k] = *reinterpret_cast<const v4f*>(p.qk_sin + (size_t)pos * half + dp);
       }
@@ -383,54 +430,52 @@ hipError_t launch_split_bf16(const float* a, int lda_f, int M, int K, __bf16* hi
   return hipGetLastError();
 }
 
-template <int BM, int BN, int NS, int AT, int BT, int WGN = 2, int BK = 32>
+template <int BM, int BN, int NS, int AT, int BT, int BK, int WGM, int WGN, int LW = 0>
 static hipError_t launch_pl(const GemmPlArgs& a, hipStream_t s) {
   const int tiles = ceil_div(a.M, BM) * ceil_div(a.N, BN);
   if (is_glu(a.act))
-    timed_launch((gemm_planes_kernel<BM, BN, NS, AT, BT, true, WGN, BK>), dim3(tiles),
-                 dim3(128 * WGN), 0, s, a);
+    timed_launch((gemm_planes_kernel<BM, BN, NS, AT, BT, true, BK, WGM, WGN, LW>), dim3(tiles),
+                 dim3(64 * (WGM * WGN + LW)), 0, s, a);
   else
-    timed_launch((gemm_planes_kernel<BM, BN, NS, AT, BT, false, WGN, BK>), dim3(tiles),
-                 dim3(128 * WGN), 0, s, a);
+    timed_launch((gemm_planes_kernel<BM, BN, NS, AT, BT, false, BK, WGM, WGN, LW>), dim3(tiles),
+                 dim3(64 * (WGM * WGN + LW)), 0, s, a);
   return hipGetLastError();
 }
 
-// Tiles: 1 = 256x256, 2 = 256x128, 3 = 128x128 with 4 waves (2x2); 4 =
-// 256x256 and 5 = 256x128 with 8 waves (2x4, two per SIMD); for one
-// activation term and int8 weights also 6 = 256x256 and 7 = 256x128 on
-// 128-byte stages (two and three); 8 = 64x64 and 9 = 128x64 with 4 waves;
-// 10 = 128x256 with 8 waves on three 64-byte stages (72 KiB: two workgroups
-// per CU), for one term.
-// Stages: as many as fit in 160 KiB of LDS. fp32's four planes leave no room
-// for 256x256 (1 and 4 fall back to 2 and 5). Automatic choice (measured on
-// MI355X at M = 16384 over the Qwen3/BERT linears; 8 waves 2-15% faster than
-// 4 at the same tile): tile 6 for one-term W8 when the 256x256 grid gives
-// at least every other CU a workgroup, 4 for the other products when it
-// gives every CU one, else 5 down to 96 tiles, else 128x128
-// while its grid has at least 192 workgroups; below that (MiniLM's M ~ 2300,
-// or N = 384) 64x64, which keeps the CUs busy: at M = 2304 the weight-only
-// int8 linears take 9.8 / 5.6 / 11.6 µs (384x1152, 384x384, 1536x384)
-// against 10.6 / 9.5 / 20.0 with 128x128.
-int pick_planes_tile(int M, int N, int K, int a_terms, int b_terms) {
-  // one term: at M = 16384, K = 3072, N = 768 the 192 tiles of tile 6 take
-  // 91 µs against 120 for the 384 tiles of 256x128
-  if (a_terms == 1 && b_terms == 1 && ceil_div(M, 256) * ceil_div(N, 256) >= 128) {
-    // Past one round, with the last round at most half full and a short K,
-    // tile 6's tail is one 256x256 workgroup per busy CU; the 128x256 tile
-    // with two workgroups per CU halves it. K = 768: M = 24576, N = 768
-    // (1.125 rounds) 47.9 against 56.1 µs; M = 16384, N = 1280 (1.25) 48.5
-    // against 57.4; N = 2304 (2.25) 84.4 against 89.1. At 1.875 rounds, whole
-    // rounds, below one round and K = 2048 tile 6 stays ahead.
-    const int t6 = ceil_div(M, 256) * ceil_div(N, 256), tail = t6 % 256;
-    return t6 > 256 && tail != 0 && tail <= 128 && K <= 1536 ? 10 : 6;
+// Tiles: 1, 4 and 6 = 256x256, 2, 5 and 7 = 256x128, 3 = 128x128, 8 = 64x64,
+// 9 = 128x64, 10 = 128x256 (one term; else 128x128). All 32-bit sums run over K
+// in the same order, so a row has the same bits on every tile.
+//
+// One term: 128x128 with two workgroups of eight waves per CU is ahead on every
+// grid that fills half the chip (weight-only int8, µs, before -> now: M = 16384,
+// K = 768: N = 768 32.4 -> 28.0, N = 2304 90.8 -> 72.7; M = 5003, N = 768 19.5 ->
+// 13.2; M = 3896, K = 2048, N = 1024 39.7 -> 25.8; M = 1213, N = 3072 19.8 ->
+// 13.3), 64x64 below (M = 349, K = 3072, N = 768 18.8 -> 14.5; at M = 2408,
+// K = 384, N = 1152, 171 tiles, 10.2 against 9.0 on 128x128; at M = 349,
+// N = 3072, 72 tiles, 9.0 against 11.2).
+// fp32: rounds of the chip times a tile's time per round in units of 1e-8 s per
+// k (256x256 86, 256x128 47.8 and 128x128 27.5 with one workgroup per CU, 64x64 8
+// with two; measured at M = 16384, K = 1024, N = 6144). µs before -> now:
+// M = 16384 620 -> 586, M = 3896, K = 3072, N = 1024 113 -> 71, M = 4012,
+// K = 1152, N = 768 46.5 -> 26.9, M = 2408, K = 1536, N = 384 17.4 -> 15.1,
+// M = 349, K = 3072, N = 768 28.5 -> 23.4.
+// Weight-only int8 on two activation terms: 256x256 while its grid fills the
+// chip, 256x128 down to 96 tiles, 128x128 down to 192, then 64x64.
+int pick_planes_tile(int M, int N, int a_terms, int b_terms) {
+  auto tiles = [&](int bm, int bn) { return (long long)ceil_div(M, bm) * ceil_div(N, bn); };
+  if (a_terms == 1 && b_terms == 1) return tiles(128, 128) >= 128 ? 3 : 8;
+  if (b_terms == 1) {
+    if (tiles(256, 256) >= 256) return 1;
+    if (tiles(256, 128) >= 96) return 2;
+    return tiles(128, 128) >= 192 ? 3 : 8;
   }
-  if (a_terms + b_terms < 4 && ceil_div(M, 256) * ceil_div(N, 256) >= 256) return 4;
-  // 256x128 down to 96 tiles (fp32 at M = 10102, N = 768: 240 tiles, 43.5 /
-  // 154 µs at K = 768 / 3072 against 53.6 / 190 on 128x128; the two-stream
-  // fp32 BERT-base forward's parts, ~5050 rows, give 120 tiles at N = 768:
-  // 1.49 against 1.41 M tokens/s end to end with 128x128 there)
-  if (ceil_div(M, 256) * ceil_div(N, 128) >= 96) return 5;
-  return ceil_div(M, 128) * ceil_div(N, 128) >= 192 ? 3 : 8;
+  const double t1 = 86.0 * ((tiles(256, 256) + 255) / 256);
+  const double t2 = 47.8 * ((tiles(256, 128) + 255) / 256);
+  const double t3 = 27.5 * ((tiles(128, 128) + 255) / 256);
+  const double t8 = 16.0 * ((tiles(64, 64) + 511) / 512);
+  if (t8 <= t1 && t8 <= t2 && t8 <= t3) return 8;
+  if (t3 <= t1 && t3 <= t2) return 3;
+  return t2 <= t1 ? 2 : 1;
 }
 
 hipError_t launch_gemm_planes_qk(const GemmPlArgs& a, hipStream_t s) {
@@ -438,8 +483,8 @@ hipError_t launch_gemm_planes_qk(const GemmPlArgs& a, hipStream_t s) {
   if (a.N % 256 != 0 || a.lda % 64 != 0 || a.ldb % 64 != 0 || a.ldc % 4 != 0 || !a.qk_out ||
       !(a.qk_dh == 64 || a.qk_dh == 128 || a.qk_dh == 256) || is_glu(a.act))
     return hipErrorInvalidValue;
-  const int tiles = ceil_div(a.M, 256) * (a.N / 256);
-  timed_launch((gemm_planes_kernel<256, 256, 2, 1, 1, false, 4, 64, true>), dim3(tiles),
+  const int tiles = ceil_div(a.M, 128) * (a.N / 256);
+  timed_launch((gemm_planes_kernel<128, 256, 3, 1, 1, false, 32, 2, 4, 0, true>), dim3(tiles),
                dim3(512), 0, s, a);
   return hipGetLastError();
 }
@@ -469,42 +514,51 @@ hipError_t launch_gemm_planes(const GemmPlArgs& a, int a_terms, int b_terms, int
       g.epi = a.Ch ? EPI_PLANES : EPI_F32;
       return launch_gemm_small_planes(g, a_terms, b_terms, small, s);
     }
-    tile = pick_planes_tile(a.M, a.N, a.K, a_terms, b_terms);
+    tile = pick_planes_tile(a.M, a.N, a_terms, b_terms);
   }
   if (a_terms == 1 && b_terms == 1) {
     switch (tile) {
-      case 1: return launch_pl<256, 256, 4, 1, 1>(a, s);
-      case 2: return launch_pl<256, 128, 4, 1, 1>(a, s);
-      case 4: return launch_pl<256, 256, 4, 1, 1, 4>(a, s);
-      case 5: return launch_pl<256, 128, 4, 1, 1, 4>(a, s);
-      case 6: return launch_pl<256, 256, 2, 1, 1, 4, 64>(a, s);
-      case 7: return launch_pl<256, 128, 3, 1, 1, 4, 64>(a, s);
-      case 8: return launch_pl<64, 64, 4, 1, 1>(a, s);
-      case 9: return launch_pl<128, 64, 4, 1, 1>(a, s);
-      case 10: return launch_pl<128, 256, 3, 1, 1, 4>(a, s);
-      default: return launch_pl<128, 128, 4, 1, 1>(a, s);
+      case 1:
+      case 4:
+      case 6: return launch_pl<256, 256, 2, 1, 1, 64, 2, 4>(a, s);
+      case 2:
+      case 5:
+      case 7: return launch_pl<256, 128, 3, 1, 1, 32, 4, 2>(a, s);
+      case 8: return launch_pl<64, 64, 4, 1, 1, 64, 2, 2, 4>(a, s);
+      case 9: return launch_pl<128, 64, 2, 1, 1, 64, 2, 2>(a, s);
+      case 10: return launch_pl<128, 256, 3, 1, 1, 32, 2, 4>(a, s);
+      default: return launch_pl<128, 128, 2, 1, 1, 64, 4, 2>(a, s);
     }
   }
   if (a_terms == 2 && b_terms == 1) {
     switch (tile) {
-      case 1: return launch_pl<256, 256, 3, 2, 1>(a, s);
-      case 2: return launch_pl<256, 128, 4, 2, 1>(a, s);
-      case 4: return launch_pl<256, 256, 3, 2, 1, 4>(a, s);
-      case 5: return launch_pl<256, 128, 4, 2, 1, 4>(a, s);
-      case 8: return launch_pl<64, 64, 4, 2, 1>(a, s);
-      case 9: return launch_pl<128, 64, 4, 2, 1>(a, s);
-      default: return launch_pl<128, 128, 3, 2, 1>(a, s);
+      case 1:
+      case 4:
+      case 6: return launch_pl<256, 256, 3, 2, 1, 32, 2, 4>(a, s);
+      case 2:
+      case 5:
+      case 7: return launch_pl<256, 128, 4, 2, 1, 32, 4, 2>(a, s);
+      case 8: return launch_pl<64, 64, 3, 2, 1, 64, 2, 2, 4>(a, s);
+      case 9: return launch_pl<128, 64, 4, 2, 1, 32, 2, 2>(a, s);
+      default: return launch_pl<128, 128, 3, 2, 1, 32, 4, 2>(a, s);
     }
   }
   if (a_terms == 2 && b_terms == 2) {
     switch (tile) {
       case 1:
-      case 2: return launch_pl<256, 128, 3, 2, 2>(a, s);
       case 4:
-      case 5: return launch_pl<256, 128, 3, 2, 2, 4>(a, s);
-      case 8: return launch_pl<64, 64, 4, 2, 2>(a, s);
-      case 9: return launch_pl<128, 64, 4, 2, 2>(a, s);
-      default: return launch_pl<128, 128, 3, 2, 2>(a, s);
+      case 6: return launch_pl<256, 256, 2, 2, 2, 32, 2, 4>(a, s);
+      case 2:
+      case 5:
+      case 7: return launch_pl<256, 128, 3, 2, 2, 32, 4, 2>(a, s);
+      case 8:  // four stages in flight with one workgroup per CU, else two with two
+        // (M = 349, K = 3072, N = 768, 72 tiles: 23.4 against 31.8; M = 349, K = 768,
+        // N = 3072, 288 tiles: 16.1 against 12.8)
+        if ((long long)ceil_div(a.M, 64) * ceil_div(a.N, 64) <= 256)
+          return launch_pl<64, 64, 4, 2, 2, 64, 2, 2, 4>(a, s);
+        return launch_pl<64, 64, 2, 2, 2, 64, 2, 2, 4>(a, s);
+      case 9: return launch_pl<128, 64, 3, 2, 2, 64, 2, 2, 4>(a, s);
+      default: return launch_pl<128, 128, 2, 2, 2, 64, 4, 2>(a, s);
     }
   }
   return hipErrorInvalidValue;

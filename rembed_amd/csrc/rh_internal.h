@@ -265,8 +265,8 @@ constexpr int kPlanesTileConfigs = 10;
 hipError_t launch_gemm_planes(const GemmPlArgs& a, int a_terms, int b_terms, int tile,
                               hipStream_t s);
 // The q|k|v projection with the QK-norm + RoPE epilogue (a.qk_out set): one
-// activation term, int8 weights as one bf16 plane, 256x256 tiles of 8 waves
-// on two 128-byte stages; needs N % 256 == 0 and qk_dh in {64, 128, 256}.
+// activation term, int8 weights as one bf16 plane, 128x256 tiles of 8 waves,
+// two workgroups per CU; needs N % 256 == 0 and qk_dh in {64, 128, 256}.
 hipError_t launch_gemm_planes_qk(const GemmPlArgs& a, hipStream_t s);
 
 // fp32 GEMM strategies (selected per model/context; both kept so the

@@ -176,3 +176,37 @@ def test_planes_vs_inloop_linear_gelu(gpu_ctx, mode, mkn):
         say(f"  bf_algo {bf}: max err {err.max():.3e} worst err/bound {(err / b).max():.3f}")
         assert np.all(err <= b)
     assert np.all(np.isfinite(outs[0]))
+
+
+@pytest.mark.parametrize("k", [1, 33, 64, 65, 130, 200, 320])
+@pytest.mark.parametrize("mode,terms", [(_lib.RH_MODE_F32, 2), (_lib.RH_MODE_W8, 1),
+                                        (_lib.RH_MODE_W8, 2)], ids=["f32", "w8", "w8-2terms"])
+def test_tiles_agree_at_short_rings(gpu_ctx, mode, terms, k):
+    """Fewer, as many and more k stages than a tile's ring holds, with ragged
+    ends: every tile gives the bits of the 64x64 one, whose error is bounded by
+    the operands' rounding (one bf16 term 2^-9, two 2^-17 and the product left
+    out) and k additions in fp32."""
+    m, n = 270, 272
+    say(f"short rings mode {mode} terms {terms} k {k}")
+    rng = np.random.default_rng(k + mode + terms)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    bT = rng.standard_normal((n, k)).astype(np.float32)
+    pb = T.PackedWeight(gpu_ctx, mode, bT, k, n)
+    gpu_ctx.set_option(_lib.RH_CTX_W8_TERMS, terms)
+    got = {}
+    try:
+        for tile in (8, 1, 2, 3, 9, 10):
+            gpu_ctx.set_option(_lib.RH_CTX_BF_TILE, tile)
+            got[tile] = T.matmul_host(gpu_ctx, a, pb)
+    finally:
+        gpu_ctx.set_option(_lib.RH_CTX_BF_TILE, 0)
+        gpu_ctx.set_option(_lib.RH_CTX_W8_TERMS, 1)
+    w = bT.astype(np.float64)
+    if mode == _lib.RH_MODE_W8:
+        q, sc, _ = pb.export()
+        w = q.astype(np.float64) * sc.astype(np.float64)[:, None]
+    a64 = a.astype(np.float64)
+    eps = (2.0 ** -9 if terms == 1 else 3 * 2.0 ** -17) + (k + 2) * 2.0 ** -24
+    assert np.all(np.abs(got[8] - a64 @ w.T) <= (np.abs(a64) @ np.abs(w).T) * eps + 1e-30)
+    for tile, out in got.items():
+        assert np.array_equal(out, got[8]), tile
