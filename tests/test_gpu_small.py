@@ -93,9 +93,9 @@ def test_planes_against_float64(gpu_ctx, shape, terms, mode):
     a64 = a.astype(np.float64)
     want = a64 @ w.T
     # |error| <= sum |a||w| · (operand rounding + the fp32 sum's): one bf16 term
-    # is off by 2^-9 of a value at most, two by 2^-17 (and the dropped lo·lo
-    # product, and w's own split); K fp32 additions in any order by K · 2^-24
-    eps = 2.0 ** -9 if terms == 1 else 3 * 2.0 ** -17
+    # (8 significant bits) is off by 2^-8 of a value at most, two by 2^-16 (and the
+    # dropped lo·lo product, and w's own split); K fp32 additions in any order by K · 2^-24
+    eps = 2.0 ** -8 if terms == 1 else 3 * 2.0 ** -16
     bound = (np.abs(a64) @ np.abs(w).T) * (eps + k * 2.0 ** -24) + 1e-30
     assert np.all(np.abs(got - want) <= bound)
 
