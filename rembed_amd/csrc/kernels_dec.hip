@@ -6,6 +6,7 @@
 // One 64-lane wave owns one row (or one head of one row); rows are 16-byte
 // aligned and every width here is a multiple of 4, so rows move as float4.
 #include "gemm_common.h"
+#include "rows_common.h"
 
 namespace rh {
 
@@ -402,49 +403,81 @@ hipError_t launch_qk_norm_rope(float* qkv, int ldqkv, int m, int nq, int nkv, in
 // ---- EmbeddingGemma Dense head --------------------------------------------------------
 // applyGemmaDenseHead (gemma3.go:174-198): hid[o] = sum_i w1[o][i] * pooled[i],
 // out[o] = sum_i w2[o][i] * hid[i], each a sequential float32 sum in ascending
-// i (no FMA). One thread per (text, output) over transposed weights
-// (wT[i][o], so a wave's loads of one i are contiguous); the text's input
-// vector is staged in LDS.
-__global__ __launch_bounds__(256) void dense_matvec_kernel(const float* __restrict__ wT,
-                                                           int in, int outn,
+// i (no FMA) over transposed weights (wT[i][o]). A workgroup takes 32 outputs of
+// 8 texts: 256 rows of its weight columns at a time go through LDS (ColChunk)
+// with the texts' inputs, and half-wave h adds text h's products. Bound by the
+// chain of additions and what a CU pulls of the weights; with a text's 256
+// outputs per workgroup each of them read the weights at one CU's rate (16
+// texts: 3072 -> 768 62 -> 36 µs, 768 -> 3072 20 -> 13).
+constexpr int kDenseTexts = 8;
+__global__ __launch_bounds__(512) void dense_matvec_kernel(const float* __restrict__ wT,
+                                                           int in, int outn, int batch,
                                                            const float* __restrict__ x,
                                                            float* __restrict__ y) {
-  extern __shared__ float xs[];  // in floats
-  const int b = blockIdx.y;
-  for (int i = threadIdx.x; i < in; i += 256) xs[i] = x[(size_t)b * in + i];
-  __syncthreads();
-  const int o = blockIdx.x * 256 + threadIdx.x;
-  if (o >= outn) return;
-  const float* w = wT + o;
-  // The sum runs i = 0, 1, ... as in the reference; only the loads run
-  // ahead: two register blocks of U weights, the next block's loads in
-  // flight while the current one is summed (each thread's chain waited on
-  // every block's memory latency before).
-  constexpr int U = 32;
+  __shared__ __attribute__((aligned(16))) float w[2][kColCols * kColStride];
+  __shared__ __attribute__((aligned(16))) float xs[2][kDenseTexts][kColRows];
+  const int b0 = blockIdx.y * kDenseTexts, nb = min(kDenseTexts, batch - b0);
+  const bool loads = threadIdx.x >= 256;  // waves 4..7
+  const int tid = threadIdx.x & 255;
+  const int h = tid >> 5;  // text b0 + h
+  const int o = blockIdx.x * kColCols + (tid & 31);
+  const float* src = wT + min(o, outn - 1);
+  const int chunks = (in + kColRows - 1) / kColRows;
+  ColChunk ch;
+  float xv[kDenseTexts];
+  auto fetch = [&](int c) {
+    const int i = min(c * kColRows + tid, in - 1);
+#pragma unroll
+    for (int t = 0; t < kDenseTexts; t++) xv[t] = x[(size_t)(b0 + min(t, nb - 1)) * in + i];
+    ch.fetch(src, outn, c * kColRows, in);
+  };
+  auto stash = [&](int c) {
+    const int n = in - c * kColRows;
+    ch.stash(w[c & 1], n);
+#pragma unroll
+    for (int t = 0; t < kDenseTexts; t++) xs[c & 1][t][tid] = tid < n ? xv[t] : 0.0f;
+  };
+  if (loads) {
+    fetch(0);
+    stash(0);
+    if (chunks > 1) fetch(1);
+  }
   float acc = 0.0f;
-  int i = 0;
-  float ta[U], tb[U];
-  auto fill = [&](float (&t)[U], int i0) {
+  for (int c = 0; c < chunks; c++) {
+    __syncthreads();  // chunk c is in LDS, and chunk c - 1 has been read
+    if (loads) {
+      if (c + 1 < chunks) stash(c + 1);
+      if (c + 2 < chunks) fetch(c + 2);
+    } else if (h < nb) {
+      const float* pw = w[c & 1] + (tid & 31) * kColStride;
+      const float* px = xs[c & 1][h];
+      // whole groups of 16, a group read under the additions of the one before;
+      // products past `in` are zeros, which change no sum
+      const int n = min(kColRows, in - c * kColRows);
+      v4f a[2][4], v[2][4];
+      auto read = [&](int g, int i) {
 #pragma unroll
-    for (int e = 0; e < U; e++) t[e] = w[(size_t)(i0 + e) * outn];
-  };
-  auto sum = [&](const float (&t)[U], int i0) {
+        for (int q = 0; q < 4; q++) {
+          a[g][q] = *reinterpret_cast<const v4f*>(pw + i + 4 * q);
+          v[g][q] = *reinterpret_cast<const v4f*>(px + i + 4 * q);
+        }
+      };
+      auto add = [&](int g) {
 #pragma unroll
-    for (int e = 0; e < U; e++) acc = acc + t[e] * xs[i0 + e];
-  };
-  if (in >= U) fill(ta, 0);
-  for (; i + 2 * U <= in; i += 2 * U) {
-    fill(tb, i + U);
-    sum(ta, i);
-    if (i + 3 * U <= in) fill(ta, i + 2 * U);
-    sum(tb, i + U);
+        for (int q = 0; q < 4; q++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) acc = acc + a[g][q][e] * v[g][q][e];
+      };
+      read(0, 0);
+      for (int i = 0; i < n; i += 32) {
+        read(1, i + 16);  // at most the chunk's last group
+        add(0);
+        if (i + 32 < n) read(0, i + 32);
+        if (i + 16 < n) add(1);
+      }
+    }
   }
-  if (i + U <= in) {  // one loaded block left
-    sum(ta, i);
-    i += U;
-  }
-  for (; i < in; i++) acc = acc + w[(size_t)i * outn] * xs[i];
-  y[(size_t)b * outn + o] = acc;
+  if (!loads && h < nb && o < outn) y[(size_t)(b0 + h) * outn + o] = acc;
 }
 
 hipError_t launch_dense_head(const float* pooled, int batch, int H, int D, const float* w1T,
@@ -452,10 +485,11 @@ hipError_t launch_dense_head(const float* pooled, int batch, int H, int D, const
                              hipStream_t s) {
   if (batch <= 0) return hipSuccess;
   if ((size_t)std::max(H, D) * sizeof(float) > 64 * 1024) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(dense_matvec_kernel, dim3(ceil_div(D, 256), batch), dim3(256),
-                     H * sizeof(float), s, w1T, H, D, pooled, hid);
-  hipLaunchKernelGGL(dense_matvec_kernel, dim3(ceil_div(H, 256), batch), dim3(256),
-                     D * sizeof(float), s, w2T, D, H, hid, out);
+  const int groups = ceil_div(batch, kDenseTexts);
+  hipLaunchKernelGGL(dense_matvec_kernel, dim3(ceil_div(D, kColCols), groups), dim3(512), 0, s,
+                     w1T, H, D, batch, pooled, hid);
+  hipLaunchKernelGGL(dense_matvec_kernel, dim3(ceil_div(H, kColCols), groups), dim3(512), 0, s,
+                     w2T, D, H, batch, hid, out);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess && normalize) e = launch_l2_rows(out, batch, H, s);
   return e;

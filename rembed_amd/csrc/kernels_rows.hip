@@ -687,31 +687,99 @@ __global__ __launch_bounds__(256) void pool_kernel(const float* __restrict__ x, 
   out[(size_t)b * H + j] = v;
 }
 
-// L2Normalize (tensor.go:540-554) of each [H] row in place: float64 sum of
-// squares in column order (the squares of float32 values are exact in
-// float64; one lane adds them as the reference's loop does), scale by
-// float32(1/sqrt(sum)); an all-zero row is left as is.
-__global__ __launch_bounds__(256) void l2_rows_kernel(float* __restrict__ y, int H) {
-  __shared__ double sq[2048];
-  __shared__ float inv_s;
-  __shared__ int zero_s;
-  float* o = y + (size_t)blockIdx.x * H;
-  double sum = 0.0;
-  for (int j0 = 0; j0 < H; j0 += 2048) {  // 2048 columns at a time through LDS
-    const int n = min(2048, H - j0);
-    for (int j = threadIdx.x; j < n; j += 256) sq[j] = (double)o[j0 + j] * (double)o[j0 + j];
-    __syncthreads();
-    if (threadIdx.x == 0)
-      for (int j = 0; j < n; j++) sum = sum + sq[j];
-    __syncthreads();
+// Mean pooling of long texts: workgroup (32 columns, text), chunks of 256 rows
+// through LDS (ColChunk), one lane per column of a fifth wave adding them in row
+// order. Bound by the chain of additions. One text of 8192 rows of 768 beside one
+// of 5003: pool_kernel 114 µs, here 46 µs; sixteen of 2048
+// (100 MB, the memory's rate): 35 -> 20-27.
+__global__ __launch_bounds__(320) void pool_long_kernel(const float* __restrict__ x, int H,
+                                                        const int32_t* __restrict__ cu,
+                                                        float* __restrict__ out) {
+  __shared__ __attribute__((aligned(16))) float buf[2][kColCols * kColStride];
+  const int b = blockIdx.y;
+  const int col = blockIdx.x * kColCols + (threadIdx.x & 31);
+  const int r0 = cu[b], len = cu[b + 1] - r0;
+  const float* src = x + (size_t)r0 * H + min(col, H - 1);
+  const int chunks = (len + kColRows - 1) / kColRows;
+  const bool loads = threadIdx.x < 256;
+  ColChunk ch;
+  if (loads) {
+    ch.fetch(src, H, 0, len);
+    ch.stash(buf[0], len);
+    if (chunks > 1) ch.fetch(src, H, kColRows, len);
   }
+  float s = 0.0f;
+  for (int c = 0; c < chunks; c++) {
+    __syncthreads();  // chunk c is in LDS, and chunk c - 1 has been read
+    if (loads) {
+      if (c + 1 < chunks) ch.stash(buf[(c + 1) & 1], len - (c + 1) * kColRows);
+      if (c + 2 < chunks) ch.fetch(src, H, (c + 2) * kColRows, len);
+    } else {
+      const float* p = buf[c & 1] + (threadIdx.x & 31) * kColStride;
+      // whole groups of 32 rows, a group read under the additions of the one
+      // before; rows past the text are zeros, which change no sum
+      const int n = min(kColRows, len - c * kColRows);
+      v4f t[2][8];
+      auto read = [&](v4f (&g)[8], int i) {
+#pragma unroll
+        for (int q = 0; q < 8; q++) g[q] = *reinterpret_cast<const v4f*>(p + i + 4 * q);
+      };
+      auto add = [&](const v4f (&g)[8]) {
+#pragma unroll
+        for (int q = 0; q < 8; q++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) s += g[q][e];
+      };
+      read(t[0], 0);
+      for (int i = 0; i < n; i += 64) {
+        read(t[1], i + 32);  // at most the chunk's last group
+        add(t[0]);
+        if (i + 64 < n) read(t[0], i + 64);
+        if (i + 32 < n) add(t[1]);
+      }
+    }
+  }
+  if (threadIdx.x >= 256 && threadIdx.x < 256 + kColCols && col < H)
+    out[(size_t)b * H + col] = s * (1.0f / (float)len);
+}
+
+// The scale of L2Normalize (tensor.go:540-554): float32(1/sqrt(S)), S the
+// float64 sum of the row's squares (exact in float64) in column order; 1 for an
+// all-zero row. Every thread gets it. The chain of H additions took 6 µs at H =
+// 768, so the squares (`part`: this thread's) are added as a tree first: both
+// sums of H nonnegative terms are within H·2^-53 of the true one, relatively, and
+// rounding, 1/x and sqrt are monotonic, so where the ends of that range give one
+// float32 scale it is the chain's. Elsewhere (or with a NaN) one thread walks the
+// chain over at(0..H-1).
+template <class F>
+__device__ __forceinline__ float l2_scale(double part, int H, F&& at) {
+  __shared__ double red[16];
+  __shared__ float inv_s;
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) part += __shfl_xor(part, o, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = part;
+  __syncthreads();
+  double sum = 0.0;
+  for (int w = 0; w < (int)(blockDim.x >> 6); w++) sum += red[w];
+  if (sum == 0.0) return 1.0f;  // no square of a float32 underflows in float64
+  const double d = (double)(H + 8) * 0x1p-51;
+  const float lo = (float)(1.0 / sqrt(sum + sum * d)), hi = (float)(1.0 / sqrt(sum - sum * d));
+  if (lo == hi) return lo;
   if (threadIdx.x == 0) {
-    zero_s = sum == 0.0;
-    inv_s = (float)(1.0 / sqrt(sum));
+    double s = 0.0;
+    for (int j = 0; j < H; j++) s = s + (double)at(j) * (double)at(j);
+    inv_s = (float)(1.0 / sqrt(s));
   }
   __syncthreads();
-  if (zero_s) return;
-  const float inv = inv_s;
+  return inv_s;
+}
+
+// L2Normalize of each [H] row in place.
+__global__ __launch_bounds__(256) void l2_rows_kernel(float* __restrict__ y, int H) {
+  float* o = y + (size_t)blockIdx.x * H;
+  double part = 0.0;
+  for (int j = threadIdx.x; j < H; j += 256) part += (double)o[j] * (double)o[j];
+  const float inv = l2_scale(part, H, [&](int j) { return o[j]; });
   for (int j = threadIdx.x; j < H; j += 256) o[j] = o[j] * inv;
 }
 
@@ -721,11 +789,64 @@ hipError_t launch_l2_rows(float* y, int rows, int H, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_pool(const float* x, int H, const int32_t* cu, int batch,
+// Pooling and L2Normalize of one text per workgroup (H <= 2048: two columns per
+// thread), for short texts and CLS / last-token pooling: the arithmetic of
+// pool_kernel and l2_rows_kernel without the launch between them.
+__global__ __launch_bounds__(1024) void pool_l2_kernel(const float* __restrict__ x, int H,
+                                                       const int32_t* __restrict__ cu, int pooling,
+                                                       float* __restrict__ out) {
+  __shared__ float row[2048];
+  const int b = blockIdx.x;
+  const int r0 = cu[b], len = cu[b + 1] - r0;
+  float v[2] = {0.0f, 0.0f};
+  double part = 0.0;
+#pragma unroll
+  for (int k = 0; k < 2; k++) {
+    const int j = threadIdx.x + 1024 * k;
+    if (j >= H) continue;
+    if (pooling == RH_POOL_MEAN) {
+      const float* col = x + (size_t)r0 * H + j;
+      float s = 0.0f;
+      for (int i = 0; i < len; i += 16) {
+        float t[16];
+#pragma unroll
+        for (int e = 0; e < 16; e++) t[e] = col[(size_t)min(i + e, len - 1) * H];
+#pragma unroll
+        for (int e = 0; e < 16; e++) s += i + e < len ? t[e] : 0.0f;  // + 0 changes no sum
+      }
+      v[k] = s * (1.0f / (float)len);
+    } else {
+      v[k] = x[(size_t)(pooling == RH_POOL_CLS ? r0 : r0 + len - 1) * H + j];
+    }
+    row[j] = v[k];
+    part += (double)v[k] * (double)v[k];
+  }
+  const float inv = l2_scale(part, H, [&](int j) { return row[j]; });
+#pragma unroll
+  for (int k = 0; k < 2; k++) {
+    const int j = threadIdx.x + 1024 * k;
+    if (j < H) out[(size_t)b * H + j] = v[k] * inv;
+  }
+}
+
+// max_len: at least every text's length. Which kernel: see each; mean pooling
+// goes by the longest text (one workgroup adds up to 64 rows of a text while the
+// launch that it saves would take; past 512 rows pool_kernel's columns wait for
+// what three CUs per text can load).
+hipError_t launch_pool(const float* x, int H, const int32_t* cu, int batch, int max_len,
                        int pooling, int normalize, float* out, hipStream_t s) {
   if (batch <= 0) return hipSuccess;
-  hipLaunchKernelGGL(pool_kernel, dim3(ceil_div(H, 256), batch), dim3(256), 0, s, x, H, cu,
-                     pooling, out);
+  const bool mean = pooling == RH_POOL_MEAN;
+  if (normalize && H <= 2048 && (!mean || max_len <= 64)) {
+    hipLaunchKernelGGL(pool_l2_kernel, dim3(batch), dim3(1024), 0, s, x, H, cu, pooling, out);
+    return hipGetLastError();
+  }
+  if (mean && max_len > 512)
+    hipLaunchKernelGGL(pool_long_kernel, dim3(ceil_div(H, kColCols), batch), dim3(320), 0, s, x, H,
+                       cu, out);
+  else
+    hipLaunchKernelGGL(pool_kernel, dim3(ceil_div(H, 256), batch), dim3(256), 0, s, x, H, cu,
+                       pooling, out);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess && normalize) e = launch_l2_rows(out, batch, H, s);
   return e;

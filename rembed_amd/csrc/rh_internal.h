@@ -358,7 +358,7 @@ hipError_t launch_layernorm(float* x, const float* gamma, const float* beta,
                             int m, int H, float eps, hipStream_t s);
 
 // pooling + optional L2 per text (bert.go:669-703, tensor.go:542-554)
-hipError_t launch_pool(const float* x, int H, const int32_t* cu, int batch,
+hipError_t launch_pool(const float* x, int H, const int32_t* cu, int batch, int max_len,
                        int pooling, int normalize, float* out, hipStream_t s);
 
 // Multi-head attention over a packed varlen batch (bert.go:853-902 per

@@ -5,12 +5,16 @@ with a ragged last one (and grids that send a mode to its next tile or to the
 tiled kernels), K one element, less than one 64-byte step, steps that leave
 waves without a share, ragged ends and the deep linears.
 """
+import dataclasses
+
 import numpy as np
 import pytest
 
 from oracle import oracle as O
 from rembed_amd import _lib
 from rembed_amd import tensor as T
+from rembed_amd.model import Model
+from rembed_amd.synthetic import GEMMA3_300M, BertShape, bert_tensors, decoder_tensors
 
 pytestmark = pytest.mark.gpu
 
@@ -179,3 +183,57 @@ def test_row_kernels_few_and_many_rows_agree(gpu_ctx, n):
     assert np.array_equal(ln[2048][:1], ln[1]) and np.array_equal(ln[m][:2048], ln[2048])
     assert np.array_equal(qs[2048][:1], qs[1]) and np.array_equal(qs[m][:2048], qs[2048])
     assert np.array_equal(qs[m], np.stack([O.quantize_row_u8(r)[0] for r in x]))
+
+
+def in_order(terms, dtype):
+    """The rows of `terms` added one after the other in dtype, from zero."""
+    return np.cumsum(np.concatenate([np.zeros_like(terms[:1]), terms]), axis=0, dtype=dtype)[-1]
+
+
+def l2(v):
+    s = in_order(np.square(v.astype(np.float64)), np.float64)
+    return v if s == 0 else v * np.float32(1.0 / np.sqrt(s))
+
+
+@pytest.mark.parametrize("pooling", [0, 1, 2])
+@pytest.mark.parametrize("lens", [[1], [64, 63, 1], [65, 2], [512, 31, 300], [513, 1, 256, 257, 512],
+                                  [1030, 768, 33]])
+def test_pooling_in_row_order(gpu_ctx, lens, pooling):
+    """Mean (float32, row after row), CLS and last-token pooling and the L2 scale
+    of the longest texts of each kernel and one more, bit for bit from the token
+    vectors of the same forward."""
+    say(f"pooling {pooling} lens={lens}")
+    shape = BertShape("pool", layers=1, hidden=192, heads=6, intermediate=320, vocab=500,
+                      max_position=1032, pooling=pooling, normalize=1)
+    m = Model(gpu_ctx, shape, bert_tensors(shape, seed=3), 0)
+    rng = np.random.default_rng(len(lens) + pooling)
+    ids = rng.integers(0, shape.vocab, (len(lens), max(lens)))
+    lens = np.array(lens, np.int32)
+    got, tokens = m.embed(ids, lens), m.embed_tokens(ids, lens)
+    for b, t in enumerate(tokens):
+        v = {0: lambda: in_order(t, np.float32) * (np.float32(1) / np.float32(len(t))),
+             1: lambda: t[0], 2: lambda: t[-1]}[pooling]()
+        assert np.array_equal(got[b], l2(v)), b
+
+
+@pytest.mark.parametrize("batch", [1, 3, 8, 9])
+@pytest.mark.parametrize("dense", [32, 300, 1056])
+def test_dense_head_in_order(gpu_ctx, batch, dense):
+    """EmbeddingGemma's two head products, each output one float32 sum in
+    ascending order, bit for bit from the token vectors; widths that leave
+    ragged chunks and column tiles, batches around a workgroup's 8 texts."""
+    say(f"dense head batch={batch} dense={dense}")
+    shape = dataclasses.replace(GEMMA3_300M, name="head", layers=1, sliding_pattern=1, vocab=500,
+                                dense_hidden=dense)
+    t = decoder_tensors(shape, seed=5)
+    m = Model(gpu_ctx, shape, t, 0)
+    rng = np.random.default_rng(batch + dense)
+    lens = rng.integers(1, 40, batch).astype(np.int32)
+    ids = rng.integers(0, shape.vocab, (batch, int(lens.max())))
+    got, tokens = m.embed(ids, lens), m.embed_tokens(ids, lens)
+    w1, w2 = t["2_Dense.linear.weight"], t["3_Dense.linear.weight"]
+    for b, x in enumerate(tokens):
+        v = in_order(x, np.float32) * (np.float32(1) / np.float32(len(x)))
+        v = in_order(w1.T * v[:, None], np.float32)
+        v = in_order(w2.T * v[:, None], np.float32)
+        assert np.array_equal(got[b], l2(v) if shape.normalize else v), b
