@@ -201,6 +201,17 @@ struct rh_model {
   // from the caller's int64); reused once the previous call has synced
   int32_t* ids_pinned = nullptr;
   size_t ids_pinned_cap = 0;
+  // ids that the next forward's upload takes along with the row offsets
+  size_t ids_staged = 0;
+  // pinned landing place of the host-buffer calls' vectors (grow-only, up to
+  // kOutStaged bytes), behind 16 bytes for the one-pass FFN1's timeout flag; each
+  // call has synchronized before returning. Past kOutParted bytes the vectors
+  // leave in kOutParts pieces, the host copying one as the next arrives.
+  static constexpr size_t kOutStaged = 8 << 20, kOutParted = 1 << 20;
+  static constexpr int kOutParts = 4;
+  unsigned* out_pinned = nullptr;
+  size_t out_pinned_cap = 0;
+  hipEvent_t ev_out[kOutParts] = {};
   std::vector<int32_t> cu_host;  // packed row offsets of the current call
   // Owner of the weights above once finalized, shared with every handle
   // made by rh_model_share; null while the model is being built.
@@ -270,6 +281,13 @@ struct rh_model {
     if (ids_pinned) (void)hipHostFree(ids_pinned);
     ids_pinned = nullptr;
     ids_pinned_cap = 0;
+    if (out_pinned) (void)hipHostFree(out_pinned);
+    out_pinned = nullptr;
+    out_pinned_cap = 0;
+    for (hipEvent_t& e : ev_out) {
+      if (e) (void)hipEventDestroy(e);
+      e = nullptr;
+    }
     if (cu_evt) (void)hipEventDestroy(cu_evt);
     cu_evt = nullptr;
   }
@@ -441,6 +459,31 @@ struct rh_model {
     return RH_OK;
   }
 
+  // The pinned landing place of `bytes` vectors and the events of its parts.
+  int ensure_out_staging(size_t bytes, int parts) {
+    if (!out_pinned || bytes > out_pinned_cap) {
+      if (out_pinned) RH_HIP(hipHostFree(out_pinned));
+      out_pinned = nullptr;
+      out_pinned_cap = 0;
+      const size_t cap = round_up(std::max<size_t>(bytes, 1), 1 << 16);
+      RH_HIP(hipHostMalloc((void**)&out_pinned, 16 + cap));
+      out_pinned_cap = cap;
+    }
+    for (int p = 0; p < parts && parts > 1; p++)
+      if (!ev_out[p]) RH_HIP(hipEventCreateWithFlags(&ev_out[p], hipEventDisableTiming));
+    return RH_OK;
+  }
+
+  // The call's row offsets, and the staged ids if any, to the device. The pinned
+  // row offsets are reused once the kernel that read them before has run.
+  int upload(const std::vector<int32_t>& cu, hipStream_t s) {
+    RH_HIP(hipEventSynchronize(cu_evt));
+    memcpy(cu_pinned, cu.data(), cu.size() * sizeof(int32_t));
+    RH_HIP(launch_stage_in(cu_pinned, cu_d, (int)cu.size(), ids_pinned, ids_d, ids_staged, s));
+    RH_HIP(hipEventRecord(cu_evt, s));
+    return RH_OK;
+  }
+
   // Validate lengths (bert.go:741-747) and build packed row offsets.
   int plan(const int32_t* lens, int batch, std::vector<int32_t>& cu, int* max_len) {
     cu.assign(batch + 1, 0);
@@ -597,12 +640,7 @@ int rh_model::forward(const int32_t* ids_dev, int stride, const std::vector<int3
   const int M = cu[batch];
   int st = ensure_ws(M, batch, 0);
   if (st) return st;
-  // Row offsets: reuse the pinned buffer once its previous copy finished.
-  RH_HIP(hipEventSynchronize(cu_evt));
-  memcpy(cu_pinned, cu.data(), (batch + 1) * sizeof(int32_t));
-  RH_HIP(hipMemcpyAsync(cu_d, cu_pinned, (batch + 1) * sizeof(int32_t),
-                        hipMemcpyHostToDevice, s));
-  RH_HIP(hipEventRecord(cu_evt, s));
+  if ((st = upload(cu, s))) return st;
   if (!use_graph || ctx->profiling || !bert_no_ws())
     return forward_bert(ids_dev, stride, cu, max_len, pool, out_dev);
   if (graph.exec && graph.cu == cu && graph.ids == ids_dev && graph.stride == stride &&
@@ -927,11 +965,7 @@ int rh_model::forward_dec(const int32_t* ids_dev, int stride, const std::vector<
   const int qd = qdim(), kvd = kvdim(), qkvw = qkv_width();
   int st = ensure_ws(M, batch, 0);
   if (st) return st;
-  RH_HIP(hipEventSynchronize(cu_evt));
-  memcpy(cu_pinned, cu.data(), (batch + 1) * sizeof(int32_t));
-  RH_HIP(hipMemcpyAsync(cu_d, cu_pinned, (batch + 1) * sizeof(int32_t),
-                        hipMemcpyHostToDevice, s));
-  RH_HIP(hipEventRecord(cu_evt, s));
+  if ((st = upload(cu, s))) return st;
 
   const float emb_scale = gemma() ? (float)std::sqrt((double)H) : 1.0f;
   // nomic adds the segment-0 row (type0 is null for the others)
@@ -1928,25 +1962,52 @@ static int embed_common(rh_model* m, const int64_t* ids, const int32_t* lens, in
     for (int t = lens[b]; t < stride; t++) srow[t] = 0;  // never read
   }
   hipStream_t s = m->ctx->stream;
-  RH_HIP(hipMemcpyAsync(m->ids_d, stage, elems * sizeof(int32_t), hipMemcpyHostToDevice, s));
+  const size_t n = (size_t)(pool ? batch : M) * H, bytes = n * sizeof(float);  // H % 64 == 0
+  const bool staged = bytes <= rh_model::kOutStaged;
+  const int parts = staged && bytes > rh_model::kOutParted ? rh_model::kOutParts : 1;
+  if ((st = m->ensure_out_staging(staged ? bytes : 0, parts))) return st;
   // the staging rows are reused by the next call only after this one's sync
+  m->ids_staged = elems;
   st = m->forward(m->ids_d, stride, cu, max_len, pool, m->out_d);
+  m->ids_staged = 0;
   if (st) {
     (void)hipStreamSynchronize(s);
     return st;
   }
-  if (pool)
-    RH_HIP(hipMemcpyAsync(out, m->out_d, (size_t)batch * H * sizeof(float),
-                          hipMemcpyDeviceToHost, s));
-  else
-    RH_HIP(hipMemcpyAsync(out, m->x, (size_t)M * H * sizeof(float), hipMemcpyDeviceToHost,
-                          s));
-  // a one-pass FFN1 row wait that timed out left bytes that may be wrong
-  unsigned late = 0;
+  // The vectors go through the pinned buffer (more than it holds straight to the
+  // caller's) with, for one-pass FFN1s, the flag of a row wait that timed out and
+  // left bytes that may be wrong.
+  const float* vec = pool ? m->out_d : m->x;
+  float* land = reinterpret_cast<float*>(m->out_pinned + 4);
   const bool onepass = m->qsync && m->fused_ffn1 == 2;
-  if (onepass) RH_HIP(hipMemcpyAsync(&late, m->qsync, sizeof(unsigned), hipMemcpyDeviceToHost, s));
-  RH_HIP(hipStreamSynchronize(s));
-  if (late) {
+  m->out_pinned[0] = 0;
+  hipError_t e = hipSuccess;
+  auto part_end = [&](int p) { return p + 1 == parts ? n : n / parts * (p + 1) / 64 * 64; };
+  size_t at = 0;
+  for (int p = 0; p < parts && e == hipSuccess; p++) {
+    const size_t end = part_end(p);
+    e = launch_stage_out(vec + at, land + at, staged ? end - at : 0, onepass ? m->qsync : nullptr,
+                         m->out_pinned, s);
+    if (e == hipSuccess && parts > 1) e = hipEventRecord(m->ev_out[p], s);
+    at = end;
+  }
+  // Touch the caller's pages while the forward runs: a fresh buffer's page faults
+  // would otherwise stand in the copies.
+  if (bytes >= 1 << 16)
+    for (size_t i = 0; i < bytes; i += 4096) reinterpret_cast<volatile char*>(out)[i] = 0;
+  if (e == hipSuccess && !staged) e = hipMemcpyAsync(out, vec, bytes, hipMemcpyDeviceToHost, s);
+  at = 0;
+  for (int p = 0; p + 1 < parts && e == hipSuccess; p++) {
+    const size_t end = part_end(p);
+    e = hipEventSynchronize(m->ev_out[p]);
+    if (e == hipSuccess) memcpy(out + at, land + at, (end - at) * sizeof(float));
+    at = end;
+  }
+  const hipError_t es = hipStreamSynchronize(s);
+  if (e != hipSuccess) return hip_fail(e, "output copy", __FILE__, __LINE__);
+  RH_HIP(es);
+  if (staged) memcpy(out + at, land + at, (n - at) * sizeof(float));
+  if (m->out_pinned[0]) {
     RH_HIP(hipMemset(m->qsync, 0, sizeof(unsigned)));
     return fail(RH_ERR_HIP, "one-pass FFN1: a row's wait for its row maxima timed out");
   }

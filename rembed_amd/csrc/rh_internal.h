@@ -357,6 +357,13 @@ hipError_t launch_add_layernorm(float* x, const float* y, int ldy,
 hipError_t launch_layernorm(float* x, const float* gamma, const float* beta,
                             int m, int H, float eps, hipStream_t s);
 
+// Pinned host memory to and from the device by kernel, in stream order: ncu row
+// offsets and n ids in; n floats (a multiple of 4) and, if given, a flag word out.
+hipError_t launch_stage_in(const int32_t* cu_h, int32_t* cu, int ncu, const int32_t* ids_h,
+                           int32_t* ids, size_t n, hipStream_t s);
+hipError_t launch_stage_out(const float* src, float* dst_h, size_t n, const unsigned* flag,
+                            unsigned* flag_h, hipStream_t s);
+
 // pooling + optional L2 per text (bert.go:669-703, tensor.go:542-554)
 hipError_t launch_pool(const float* x, int H, const int32_t* cu, int batch, int max_len,
                        int pooling, int normalize, float* out, hipStream_t s);

@@ -237,3 +237,22 @@ def test_dense_head_in_order(gpu_ctx, batch, dense):
         v = in_order(w1.T * v[:, None], np.float32)
         v = in_order(w2.T * v[:, None], np.float32)
         assert np.array_equal(got[b], l2(v) if shape.normalize else v), b
+
+
+@pytest.mark.parametrize("rows", [1, 682, 683, 700, 5461, 5462])
+def test_token_vectors_of_every_way_out(gpu_ctx, rows):
+    """Token vectors that leave through the pinned buffer in one piece (up to
+    1 MiB), in four (up to 8 MiB) and straight to the caller's memory: the same
+    bits as the texts in small calls (full int8: a row does not depend on the
+    batch it is in), and again on a second call."""
+    say(f"token vectors rows={rows}")
+    shape = BertShape("out", layers=1, hidden=384, heads=12, intermediate=384, vocab=500,
+                      max_position=512)
+    m = Model(gpu_ctx, shape, bert_tensors(shape, seed=9), 2)
+    lens = np.array([512] * (rows // 512) + ([rows % 512] if rows % 512 else []), np.int32)
+    rng = np.random.default_rng(rows)
+    ids = rng.integers(0, shape.vocab, (len(lens), 512))
+    want = [m.embed_tokens(ids[b:b + 1], lens[b:b + 1])[0] for b in range(len(lens))]
+    for _ in range(2):
+        for a, b in zip(m.embed_tokens(ids, lens), want):
+            assert np.array_equal(a, b)
