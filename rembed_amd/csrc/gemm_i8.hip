@@ -1040,21 +1040,22 @@ static hipError_t launch_epi(const GemmI8Args& a, int tile, hipStream_t s) {
 // per CU; ahead of 256x256 by 7-12% at N = 3072), or its 128-byte-stage
 // form where that occupancy cannot be had or does not pay: a grid of at
 // most one workgroup per CU (N = 768 at M = 10102) or deep K (3072), where
-// the halved barrier count wins. Small problems keep 128x128 so the grid
-// still covers the CUs.
+// the halved barrier count wins.
 int pick_i8_tile(int M, int N, int K, int epi) {
   (void)epi;
+  // 64x256 with B fragments straight to registers while its grid is one round
+  // of the chip: twice the workgroups of 128x256, half the LDS reads of the
+  // tiles without fragments (µs against the 128x256 fragment tile and 128x128;
+  // M = 1213, K = 768, N = 3072 16.4 against 18.7 and 18.3; M = 5003, N = 768:
+  // K = 768 16.4 against 19.0 and 18.6, K = 3072 27.5 against 33.3 and 35.6; the
+  // two-stream BERT-base forward of 64 documents, whose O and FFN2 run here,
+  // 3208 -> 3133)
+  if (ceil_div(M, 64) * ceil_div(N, 256) <= 256) return 11;
   const int tiles = ceil_div(M, 128) * ceil_div(N, 256);
-  // The fragment-B 128x256 tile (B fragments straight to registers halve
-  // the LDS reads) for deep K on a grid of at most one such workgroup per CU
-  // (the BERT-base FFN2 at M = 10102: 34.2 against 35.5 µs fp32 out, 31.9
-  // against 33.2 int32 out), and for any K on 64..127 of them: the
-  // two-stream headline runs its parts of ~5050 rows, where O and FFN2 give
-  // 120 such tiles; against 128x128 there the whole forward went from 3.28
-  // to 3.34 M tokens/s with FFN2 on it and from 3.47 to 3.51 with O as well
-  // (interleaved runs)
-  if ((K >= 2048 || tiles < 128) && tiles <= 256 && tiles >= 64) return 13;
-  if (tiles < 128) return 3;
+  // the fragment-B 128x256 tile for deep K on a grid of at most one such
+  // workgroup per CU (the BERT-base FFN2 at M = 10102: 34.2 against 35.5 µs
+  // fp32 out, 31.9 against 33.2 int32 out)
+  if (K >= 2048 && tiles <= 256) return 13;
   // deep K on a grid of at least one 256x256 tile per CU: the 128x128-wave
   // tile (4-12 % ahead of tiles 7 and 9 at M = 16384, K = 2048 and 3072)
   const int nk = ceil_div(K, 64);
@@ -1112,7 +1113,8 @@ hipError_t launch_gemm_i8(const GemmI8Args& a, int tile, hipStream_t s) {
       return launch_gemm_small_i8(g, small, s);
     }
     tile = pick_i8_tile(a.M, a.N, a.K, a.epi);
-    if (tile == 13 && !a.Bf) tile = 9;  // no fragment-ordered image of B
+    if (!a.Bf && tile == 11) tile = 3;  // no fragment-ordered image of B
+    if (!a.Bf && tile == 13) tile = 9;
   }
   switch (a.epi) {
     case EPI_F32: return launch_epi<EPI_F32>(a, tile, s);

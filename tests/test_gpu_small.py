@@ -256,3 +256,34 @@ def test_token_vectors_of_every_way_out(gpu_ctx, rows):
     for _ in range(2):
         for a, b in zip(m.embed_tokens(ids, lens), want):
             assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("act", [_lib.RH_ACT_NONE, _lib.RH_ACT_GELU, _lib.RH_ACT_SWIGLU,
+                                 _lib.RH_ACT_GEGLU_ERF])
+@pytest.mark.parametrize("shape", [(1213, 768, 3072), (1025, 200, 4128), (700, 3072, 2080),
+                                   (16300, 64, 256), (16385, 130, 288)])
+def test_int8_one_round_of_the_chip(gpu_ctx, shape, act):
+    """Grids of up to 256 64x256 tiles and just past them: integer sums and one
+    epilogue, so the bits of a forced 128x128 tile."""
+    m, k, n = shape
+    say(f"int8 one round m={m} k={k} n={n} act={act}")
+    rng = np.random.default_rng(m + k + n + act)
+    wt = (rng.standard_normal((n, k)) * 0.05).astype(np.float32)
+    gated = act not in (_lib.RH_ACT_NONE, _lib.RH_ACT_GELU)
+    if gated:
+        pb = T.PackedGated(gpu_ctx, 2, wt[: n // 2].copy(), wt[n // 2:].copy(), k, n // 2)
+    else:
+        pb = T.PackedWeight(gpu_ctx, 2, wt, k, n, rng.standard_normal(n).astype(np.float32))
+    cols, ldq = (n // 2 if gated else n), T.ldq_for(k)
+    da, dst = gpu_ctx.upload(rows(rng, m, k)), gpu_ctx.alloc(m * cols * 4)
+    qa, rs = gpu_ctx.alloc(m * ldq), gpu_ctx.alloc(m * 4)
+    out = []
+    for tile in (0, 3):
+        gpu_ctx.set_option(_lib.RH_CTX_I8_TILE, tile)
+        try:
+            T.Linear(gpu_ctx, dst, da, pb, m, act, qa, ldq, rs)
+            gpu_ctx.sync()
+        finally:
+            gpu_ctx.set_option(_lib.RH_CTX_I8_TILE, 0)
+        out.append(dst.download(np.float32, (m, cols)))
+    assert np.array_equal(out[0], out[1])
