@@ -446,24 +446,46 @@ static hipError_t launch_pl(const GemmPlArgs& a, hipStream_t s) {
 // 9 = 128x64, 10 = 128x256 (one term; else 128x128). All 32-bit sums run over K
 // in the same order, so a row has the same bits on every tile.
 //
-// One term: 128x128 with two workgroups of eight waves per CU is ahead on every
-// grid that fills half the chip (weight-only int8, µs, before -> now: M = 16384,
-// K = 768: N = 768 32.4 -> 28.0, N = 2304 90.8 -> 72.7; M = 5003, N = 768 19.5 ->
-// 13.2; M = 3896, K = 2048, N = 1024 39.7 -> 25.8; M = 1213, N = 3072 19.8 ->
-// 13.3), 64x64 below (M = 349, K = 3072, N = 768 18.8 -> 14.5; at M = 2408,
-// K = 384, N = 1152, 171 tiles, 10.2 against 9.0 on 128x128; at M = 349,
-// N = 3072, 72 tiles, 9.0 against 11.2).
-// fp32: rounds of the chip times a tile's time per round in units of 1e-8 s per
-// k (256x256 86, 256x128 47.8 and 128x128 27.5 with one workgroup per CU, 64x64 8
-// with two; measured at M = 16384, K = 1024, N = 6144). µs before -> now:
-// M = 16384 620 -> 586, M = 3896, K = 3072, N = 1024 113 -> 71, M = 4012,
-// K = 1152, N = 768 46.5 -> 26.9, M = 2408, K = 1536, N = 384 17.4 -> 15.1,
-// M = 349, K = 3072, N = 768 28.5 -> 23.4.
+// One term, fp32: the tile whose rounds of the chip take the least. One-term
+// tiles cost, in µs, c0 + full rounds * (r + rk*K) + (h + hk*K) if a last round
+// of two-per-CU tiles puts at most one workgroup on a CU (fitted to 300 sizes of
+// M 256..32768, K 200..3200, N 320..6400 on MI355X; the choice is within 0.5 % of
+// the fastest tile on average). 128x128 is ahead on up to a few rounds of short
+// K, 256x256 on many or deep ones, where its operands are read half as often
+// (weight-only int8, µs on 128x128 against 256x256: M = 32768, K = 3072, N = 1024
+// 250 - 195; M = 16384, K = 2048, N = 1024 76.9 - 66.5; M = 16384, K = 768, N = 3072
+// 101 - 91.8, N = 2304 72.7 - 89); 64x64 where they leave CUs idle (M = 2048,
+// K = 2048, N = 1024 22.8 - 17.4 on 64x64). Gated rows leave a 256x256 workgroup
+// alone on its CU for a long epilogue; 128x256, two to a CU, hides it (M = 16384,
+// K = 768, N = 6144 213 - 201).
+// fp32: as units of 1e-8 s per k (256x256 86, 256x128 47.8 and 128x128 27.5 with
+// one workgroup per CU, 64x64 8 with two; measured at M = 16384, K = 1024, N =
+// 6144). µs before -> now: M = 16384 620 -> 586, M = 3896, K = 3072, N = 1024
+// 113 -> 71, M = 4012, K = 1152, N = 768 46.5 -> 26.9, M = 2408, K = 1536, N = 384
+// 17.4 -> 15.1, M = 349, K = 3072, N = 768 28.5 -> 23.4.
 // Weight-only int8 on two activation terms: 256x256 while its grid fills the
 // chip, 256x128 down to 96 tiles, 128x128 down to 192, then 64x64.
-int pick_planes_tile(int M, int N, int a_terms, int b_terms) {
+int pick_planes_tile(int M, int N, int K, int a_terms, int b_terms, bool glu) {
   auto tiles = [&](int bm, int bn) { return (long long)ceil_div(M, bm) * ceil_div(N, bn); };
-  if (a_terms == 1 && b_terms == 1) return tiles(128, 128) >= 128 ? 3 : 8;
+  if (a_terms == 1 && b_terms == 1) {
+    auto cost = [&](long long t, int per_cu, double c0, double r, double rk, double h, double hk) {
+      const long long round = 256LL * per_cu, rest = t % round;
+      const bool half = per_cu == 2 && rest > 0 && rest <= 256;
+      const long long full = t / round + (rest > 0 && !half);
+      return c0 + full * (r + rk * K) + (half ? h + hk * K : 0.0);
+    };
+    const double t1 = cost(tiles(256, 256), 1, -2.5, glu ? 19.0 : 13.0, 0.0216, 0.0, 0.0);
+    const double t3 = cost(tiles(128, 128), 2, 1.8, glu ? 4.7 : 3.6, 0.0160, glu ? 3.7 : 2.6, 0.0076);
+    const double t8 = cost(tiles(64, 64), 2, 2.8, glu ? 2.0 : 1.6, 0.0058, glu ? 2.0 : 1.3, 0.0038);
+    int best = t1 < t3 ? 1 : 3;
+    double us = std::min(t1, t3);
+    if (t8 < us) {
+      best = 8;
+      us = t8;
+    }
+    if (glu && cost(tiles(128, 256), 2, 0.3, 7.4, 0.0310, 9.5, 0.0146) < us) best = 10;
+    return best;
+  }
   if (b_terms == 1) {
     if (tiles(256, 256) >= 256) return 1;
     if (tiles(256, 128) >= 96) return 2;
@@ -514,7 +536,7 @@ hipError_t launch_gemm_planes(const GemmPlArgs& a, int a_terms, int b_terms, int
       g.epi = a.Ch ? EPI_PLANES : EPI_F32;
       return launch_gemm_small_planes(g, a_terms, b_terms, small, s);
     }
-    tile = pick_planes_tile(a.M, a.N, a_terms, b_terms);
+    tile = pick_planes_tile(a.M, a.N, a.K, a_terms, b_terms, is_glu(a.act));
   }
   if (a_terms == 1 && b_terms == 1) {
     switch (tile) {

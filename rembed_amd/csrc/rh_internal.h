@@ -264,6 +264,7 @@ hipError_t launch_split_bf16(const float* a, int lda_f, int M, int K, __bf16* hi
 constexpr int kPlanesTileConfigs = 10;
 hipError_t launch_gemm_planes(const GemmPlArgs& a, int a_terms, int b_terms, int tile,
                               hipStream_t s);
+int pick_planes_tile(int M, int N, int K, int a_terms, int b_terms, bool glu);
 // The q|k|v projection with the QK-norm + RoPE epilogue (a.qk_out set): one
 // activation term, int8 weights as one bf16 plane, 128x256 tiles of 8 waves,
 // two workgroups per CU; needs N % 256 == 0 and qk_dh in {64, 128, 256}.
