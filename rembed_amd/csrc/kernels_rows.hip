@@ -829,19 +829,42 @@ __global__ __launch_bounds__(1024) void pool_l2_kernel(const float* __restrict__
   }
 }
 
-// max_len: at least every text's length. Which kernel: see each; mean pooling
-// goes by the longest text (one workgroup adds up to 64 rows of a text while the
-// launch that it saves would take; past 512 rows pool_kernel's columns wait for
-// what three CUs per text can load).
-hipError_t launch_pool(const float* x, int H, const int32_t* cu, int batch, int max_len,
+// Which kernel pools, and why (measured on MI355X, µs, 768 columns). One launch
+// with the L2 scale while a workgroup adds at most 64 rows of a text, the time of
+// the launch that it saves. Past 512 rows of one text pool_kernel's columns wait
+// for what three CUs per text can load, and pool_long_kernel runs where it costs
+// less: it takes a workgroup per 32 columns, and 1.3 µs a round of the chip for
+// every 256 rows of every text, which a batch of short texts beside a long one
+// does not repay (1000 texts of 5..20 and one of 520: pool_kernel 19, pool_long
+// 131; 200 of 20..100 and one of 520: 15.6 and 30; 64 of 100..300 and one of 700:
+// 21 and 14; 16 of 520: 13 and 10) nor one that is bound by the bytes (100 of
+// 300..900: 29.5 and 39).
+int pick_pool(int H, const int32_t* cu, int batch, int pooling, int normalize) {
+  const bool mean = pooling == RH_POOL_MEAN;
+  int max_len = 0, chunks = 0;
+  for (int b = 0; b < batch; b++) {
+    const int len = cu[b + 1] - cu[b];
+    max_len = std::max(max_len, len);
+    chunks += ceil_div(len, kColRows);
+  }
+  if (normalize && H <= 2048 && (!mean || max_len <= 64)) return POOL_L2;
+  if (!mean || max_len <= 512) return POOL_ROWS;
+  const double rounds = (double)chunks * ceil_div(H, kColCols) / 256;
+  const double bytes = 4.0 * (cu[batch] - cu[0]) * H;
+  const double by_chunks = std::max({3.0 + 0.005 * max_len, 4.0 + 1.3 * rounds, bytes / 3.3e6});
+  const double by_rows = 5.0 + 0.0136 * max_len + bytes / 8e6;
+  return by_chunks < by_rows ? POOL_LONG : POOL_ROWS;
+}
+
+hipError_t launch_pool(const float* x, int H, const int32_t* cu, const int32_t* cu_host, int batch,
                        int pooling, int normalize, float* out, hipStream_t s) {
   if (batch <= 0) return hipSuccess;
-  const bool mean = pooling == RH_POOL_MEAN;
-  if (normalize && H <= 2048 && (!mean || max_len <= 64)) {
+  const int kind = pick_pool(H, cu_host, batch, pooling, normalize);
+  if (kind == POOL_L2) {
     hipLaunchKernelGGL(pool_l2_kernel, dim3(batch), dim3(1024), 0, s, x, H, cu, pooling, out);
     return hipGetLastError();
   }
-  if (mean && max_len > 512)
+  if (kind == POOL_LONG)
     hipLaunchKernelGGL(pool_long_kernel, dim3(ceil_div(H, kColCols), batch), dim3(320), 0, s, x, H,
                        cu, out);
   else

@@ -941,7 +941,7 @@ int rh_model::forward_bert(const int32_t* ids_dev, int stride, const std::vector
   if (st) return st;
   if ((st = jst)) return st;
   if (pool) {
-    RH_HIP(launch_pool(x, H, cu_d, batch, max_len, cfg.pooling, cfg.normalize, out_dev, s));
+    RH_HIP(launch_pool(x, H, cu_d, cu.data(), batch, cfg.pooling, cfg.normalize, out_dev, s));
   }
   return RH_OK;
 }
@@ -1192,11 +1192,11 @@ int rh_model::forward_dec(const int32_t* ids_dev, int stride, const std::vector<
   if ((st = jst)) return st;
   if (pool) {
     if (gemma() && dense1 && dense2) {
-      RH_HIP(launch_pool(x, H, cu_d, batch, max_len, cfg.pooling, 0, pooled, s));
+      RH_HIP(launch_pool(x, H, cu_d, cu.data(), batch, cfg.pooling, 0, pooled, s));
       RH_HIP(launch_dense_head(pooled, batch, H, cfg.dense_hidden, dense1, dense2, cfg.normalize,
                                dense_hid, out_dev, s));
     } else {
-      RH_HIP(launch_pool(x, H, cu_d, batch, max_len, cfg.pooling, cfg.normalize, out_dev, s));
+      RH_HIP(launch_pool(x, H, cu_d, cu.data(), batch, cfg.pooling, cfg.normalize, out_dev, s));
     }
   }
   return RH_OK;

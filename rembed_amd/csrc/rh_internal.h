@@ -366,7 +366,10 @@ hipError_t launch_stage_out(const float* src, float* dst_h, size_t n, const unsi
                             unsigned* flag_h, hipStream_t s);
 
 // pooling + optional L2 per text (bert.go:669-703, tensor.go:542-554)
-hipError_t launch_pool(const float* x, int H, const int32_t* cu, int batch, int max_len,
+// cu_host: the host's copy of the row offsets cu, by which the kernel is chosen
+enum PoolKernel { POOL_ROWS, POOL_L2, POOL_LONG };
+int pick_pool(int H, const int32_t* cu, int batch, int pooling, int normalize);
+hipError_t launch_pool(const float* x, int H, const int32_t* cu, const int32_t* cu_host, int batch,
                        int pooling, int normalize, float* out, hipStream_t s);
 
 // Multi-head attention over a packed varlen batch (bert.go:853-902 per

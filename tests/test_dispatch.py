@@ -34,3 +34,27 @@ W8_TILES = [
 def test_one_term_planes_tile(m, k, n, gated, good):
     pick = rule("_ZN2rh16pick_planes_tileEiiiiib", *[ctypes.c_int] * 5, ctypes.c_bool)
     assert pick(m, n, k, 1, 1, gated) in good
+
+
+ROWS, L2, LONG = 0, 1, 2  # PoolKernel
+POOLS = [
+    # one long text among short ones, whose number decides
+    (768, [520] + [12] * 1000, ROWS), (768, [520] + [60] * 200, ROWS),
+    (768, [700] + [200] * 63, LONG), (768, [520] * 16, LONG), (768, [520], LONG),
+    (768, [2048] * 16, LONG), (768, [8192, 7049], LONG), (768, [8192] + [5] * 4000, ROWS),
+    (768, [900] + [400] * 99, ROWS), (768, [900] + [650] * 29, LONG),
+    (768, [6000] + [60] * 399, LONG), (768, [512] * 8, ROWS), (384, [64] * 40, L2), (384, [65, 3], ROWS),
+]
+
+
+@pytest.mark.parametrize("h,lens,kernel", POOLS)
+def test_mean_pooling_kernel(h, lens, kernel):
+    pick = rule("_ZN2rh9pick_poolEiPKiiii", ctypes.c_int, ctypes.c_void_p, *[ctypes.c_int] * 3)
+    cu = (ctypes.c_int * (len(lens) + 1))()
+    for b, n in enumerate(lens):
+        cu[b + 1] = cu[b] + n
+    assert pick(h, cu, len(lens), 0, 1) == kernel
+    # without the scale, and CLS pooling, never by way of the chunked kernel
+    assert pick(h, cu, len(lens), 0, 0) == (LONG if kernel == LONG else ROWS)
+    assert pick(h, cu, len(lens), 1, 1) == L2
+    assert pick(h, cu, len(lens), 1, 0) == ROWS
