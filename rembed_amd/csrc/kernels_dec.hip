@@ -404,38 +404,47 @@ hipError_t launch_qk_norm_rope(float* qkv, int ldqkv, int m, int nq, int nkv, in
 // applyGemmaDenseHead (gemma3.go:174-198): hid[o] = sum_i w1[o][i] * pooled[i],
 // out[o] = sum_i w2[o][i] * hid[i], each a sequential float32 sum in ascending
 // i (no FMA) over transposed weights (wT[i][o]). A workgroup takes 32 outputs of
-// 8 texts: 256 rows of its weight columns at a time go through LDS (ColChunk)
-// with the texts' inputs, and half-wave h adds text h's products. Bound by the
-// chain of additions and what a CU pulls of the weights; with a text's 256
-// outputs per workgroup each of them read the weights at one CU's rate (16
-// texts: 3072 -> 768 62 -> 36 µs, 768 -> 3072 20 -> 13).
-constexpr int kDenseTexts = 8;
+// 8 texts: 128 rows of its weight columns at a time go through LDS (ColChunk)
+// with the texts' inputs, and half-wave h adds text h's products, 4*G at a time.
+// Bound by the chain of additions and what a CU pulls of the weights while every
+// workgroup has a CU to itself (G = 4), by LDS reads and additions beyond, where
+// G = 2 leaves registers for two workgroups per CU (95 against 151). µs for both
+// products (768 -> 3072, 3072 -> 768) with a text's 256 outputs per workgroup,
+// with 256-row chunks and G = 4 throughout, and now:
+//   16 texts 73, 44, 45; 96 texts 110, 111, 76; 1024 texts 734, 837, 512
+constexpr int kDenseTexts = 8, kDenseRows = 128;
+template <int G>
 __global__ __launch_bounds__(512) void dense_matvec_kernel(const float* __restrict__ wT,
                                                            int in, int outn, int batch,
                                                            const float* __restrict__ x,
                                                            float* __restrict__ y) {
-  __shared__ __attribute__((aligned(16))) float w[2][kColCols * kColStride];
-  __shared__ __attribute__((aligned(16))) float xs[2][kDenseTexts][kColRows];
+  constexpr int kStride = ColChunk<kDenseRows>::kStride;
+  __shared__ __attribute__((aligned(16))) float w[2][kColCols * kStride];
+  __shared__ __attribute__((aligned(16))) float xs[2][kDenseTexts][kDenseRows];
   const int b0 = blockIdx.y * kDenseTexts, nb = min(kDenseTexts, batch - b0);
   const bool loads = threadIdx.x >= 256;  // waves 4..7
   const int tid = threadIdx.x & 255;
   const int h = tid >> 5;  // text b0 + h
   const int o = blockIdx.x * kColCols + (tid & 31);
   const float* src = wT + min(o, outn - 1);
-  const int chunks = (in + kColRows - 1) / kColRows;
-  ColChunk ch;
-  float xv[kDenseTexts];
+  const int chunks = (in + kDenseRows - 1) / kDenseRows;
+  ColChunk<kDenseRows> ch;
+  // the inputs: row tid % 128 of the texts tid / 128, 2 + tid / 128, ...
+  constexpr int kTextsEach = kDenseTexts * kDenseRows / 256;
+  const int xi = tid % kDenseRows, xt = tid / kDenseRows;
+  float xv[kTextsEach];
   auto fetch = [&](int c) {
-    const int i = min(c * kColRows + tid, in - 1);
+    const int i = min(c * kDenseRows + xi, in - 1);
 #pragma unroll
-    for (int t = 0; t < kDenseTexts; t++) xv[t] = x[(size_t)(b0 + min(t, nb - 1)) * in + i];
-    ch.fetch(src, outn, c * kColRows, in);
+    for (int t = 0; t < kTextsEach; t++)
+      xv[t] = x[(size_t)(b0 + min(2 * t + xt, nb - 1)) * in + i];
+    ch.fetch(src, outn, c * kDenseRows, in);
   };
   auto stash = [&](int c) {
-    const int n = in - c * kColRows;
+    const int n = in - c * kDenseRows;
     ch.stash(w[c & 1], n);
 #pragma unroll
-    for (int t = 0; t < kDenseTexts; t++) xs[c & 1][t][tid] = tid < n ? xv[t] : 0.0f;
+    for (int t = 0; t < kTextsEach; t++) xs[c & 1][2 * t + xt][xi] = xi < n ? xv[t] : 0.0f;
   };
   if (loads) {
     fetch(0);
@@ -449,35 +458,44 @@ __global__ __launch_bounds__(512) void dense_matvec_kernel(const float* __restri
       if (c + 1 < chunks) stash(c + 1);
       if (c + 2 < chunks) fetch(c + 2);
     } else if (h < nb) {
-      const float* pw = w[c & 1] + (tid & 31) * kColStride;
+      const float* pw = w[c & 1] + (tid & 31) * kStride;
       const float* px = xs[c & 1][h];
-      // whole groups of 16, a group read under the additions of the one before;
+      // whole groups of 4*G, a group read under the additions of the one before;
       // products past `in` are zeros, which change no sum
-      const int n = min(kColRows, in - c * kColRows);
-      v4f a[2][4], v[2][4];
+      const int n = min(kDenseRows, in - c * kDenseRows);
+      v4f a[2][G], v[2][G];
       auto read = [&](int g, int i) {
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
+        for (int q = 0; q < G; q++) {
           a[g][q] = *reinterpret_cast<const v4f*>(pw + i + 4 * q);
           v[g][q] = *reinterpret_cast<const v4f*>(px + i + 4 * q);
         }
       };
       auto add = [&](int g) {
 #pragma unroll
-        for (int q = 0; q < 4; q++)
+        for (int q = 0; q < G; q++)
 #pragma unroll
           for (int e = 0; e < 4; e++) acc = acc + a[g][q][e] * v[g][q][e];
       };
       read(0, 0);
-      for (int i = 0; i < n; i += 32) {
-        read(1, i + 16);  // at most the chunk's last group
+      for (int i = 0; i < n; i += 8 * G) {
+        read(1, i + 4 * G);  // at most the chunk's last group
         add(0);
-        if (i + 32 < n) read(0, i + 32);
-        if (i + 16 < n) add(1);
+        if (i + 8 * G < n) read(0, i + 8 * G);
+        if (i + 4 * G < n) add(1);
       }
     }
   }
   if (!loads && h < nb && o < outn) y[(size_t)(b0 + h) * outn + o] = acc;
+}
+
+static void launch_dense(const float* wT, int in, int outn, int batch, const float* x, float* y,
+                         hipStream_t s) {
+  const dim3 grid(ceil_div(outn, kColCols), ceil_div(batch, kDenseTexts));
+  if ((long long)grid.x * grid.y <= 256)
+    hipLaunchKernelGGL((dense_matvec_kernel<4>), grid, dim3(512), 0, s, wT, in, outn, batch, x, y);
+  else
+    hipLaunchKernelGGL((dense_matvec_kernel<2>), grid, dim3(512), 0, s, wT, in, outn, batch, x, y);
 }
 
 hipError_t launch_dense_head(const float* pooled, int batch, int H, int D, const float* w1T,
@@ -485,11 +503,8 @@ hipError_t launch_dense_head(const float* pooled, int batch, int H, int D, const
                              hipStream_t s) {
   if (batch <= 0) return hipSuccess;
   if ((size_t)std::max(H, D) * sizeof(float) > 64 * 1024) return hipErrorInvalidValue;
-  const int groups = ceil_div(batch, kDenseTexts);
-  hipLaunchKernelGGL(dense_matvec_kernel, dim3(ceil_div(D, kColCols), groups), dim3(512), 0, s,
-                     w1T, H, D, batch, pooled, hid);
-  hipLaunchKernelGGL(dense_matvec_kernel, dim3(ceil_div(H, kColCols), groups), dim3(512), 0, s,
-                     w2T, D, H, batch, hid, out);
+  launch_dense(w1T, H, D, batch, pooled, hid, s);
+  launch_dense(w2T, D, H, batch, hid, out, s);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess && normalize) e = launch_l2_rows(out, batch, H, s);
   return e;

@@ -687,38 +687,39 @@ __global__ __launch_bounds__(256) void pool_kernel(const float* __restrict__ x, 
   out[(size_t)b * H + j] = v;
 }
 
-// Mean pooling of long texts: workgroup (32 columns, text), chunks of 256 rows
-// through LDS (ColChunk), one lane per column of a fifth wave adding them in row
+// Mean pooling of long texts: workgroup (32 columns, text), chunks of kPoolRows
+// rows through LDS (ColChunk), one lane per column of a fifth wave adding them in row
 // order. Bound by the chain of additions. One text of 8192 rows of 768 beside one
 // of 5003: pool_kernel 114 µs, here 46 µs; sixteen of 2048
 // (100 MB, the memory's rate): 35 -> 20-27.
+constexpr int kPoolRows = 256;
 __global__ __launch_bounds__(320) void pool_long_kernel(const float* __restrict__ x, int H,
                                                         const int32_t* __restrict__ cu,
                                                         float* __restrict__ out) {
-  __shared__ __attribute__((aligned(16))) float buf[2][kColCols * kColStride];
+  __shared__ __attribute__((aligned(16))) float buf[2][kColCols * ColChunk<kPoolRows>::kStride];
   const int b = blockIdx.y;
   const int col = blockIdx.x * kColCols + (threadIdx.x & 31);
   const int r0 = cu[b], len = cu[b + 1] - r0;
   const float* src = x + (size_t)r0 * H + min(col, H - 1);
-  const int chunks = (len + kColRows - 1) / kColRows;
+  const int chunks = (len + kPoolRows - 1) / kPoolRows;
   const bool loads = threadIdx.x < 256;
-  ColChunk ch;
+  ColChunk<kPoolRows> ch;
   if (loads) {
     ch.fetch(src, H, 0, len);
     ch.stash(buf[0], len);
-    if (chunks > 1) ch.fetch(src, H, kColRows, len);
+    if (chunks > 1) ch.fetch(src, H, kPoolRows, len);
   }
   float s = 0.0f;
   for (int c = 0; c < chunks; c++) {
     __syncthreads();  // chunk c is in LDS, and chunk c - 1 has been read
     if (loads) {
-      if (c + 1 < chunks) ch.stash(buf[(c + 1) & 1], len - (c + 1) * kColRows);
-      if (c + 2 < chunks) ch.fetch(src, H, (c + 2) * kColRows, len);
+      if (c + 1 < chunks) ch.stash(buf[(c + 1) & 1], len - (c + 1) * kPoolRows);
+      if (c + 2 < chunks) ch.fetch(src, H, (c + 2) * kPoolRows, len);
     } else {
-      const float* p = buf[c & 1] + (threadIdx.x & 31) * kColStride;
+      const float* p = buf[c & 1] + (threadIdx.x & 31) * ColChunk<kPoolRows>::kStride;
       // whole groups of 32 rows, a group read under the additions of the one
       // before; rows past the text are zeros, which change no sum
-      const int n = min(kColRows, len - c * kColRows);
+      const int n = min(kPoolRows, len - c * kPoolRows);
       v4f t[2][8];
       auto read = [&](v4f (&g)[8], int i) {
 #pragma unroll
@@ -845,7 +846,7 @@ int pick_pool(int H, const int32_t* cu, int batch, int pooling, int normalize) {
   for (int b = 0; b < batch; b++) {
     const int len = cu[b + 1] - cu[b];
     max_len = std::max(max_len, len);
-    chunks += ceil_div(len, kColRows);
+    chunks += ceil_div(len, kPoolRows);
   }
   if (normalize && H <= 2048 && (!mean || max_len <= 64)) return POOL_L2;
   if (!mean || max_len <= 512) return POOL_ROWS;

@@ -112,35 +112,37 @@ __device__ __forceinline__ void ln_vec_finish(v4f (&v)[V], int lane, int row, in
 
 // Column sums in row order (mean pooling, the Dense head) are one serial chain
 // of float32 additions per column, so the rows have to reach the adding lane
-// ahead of it. A workgroup takes 32 columns: 256 threads load chunks of 256 rows
+// ahead of it. A workgroup takes 32 columns: 256 threads load chunks of ROWS rows
 // (128-byte row pieces) two chunks ahead and park them in LDS by column, where
 // the adding lanes, of other waves, read 4 consecutive rows at a time.
-constexpr int kColCols = 32, kColRows = 256, kColStride = kColRows + 4;
+constexpr int kColCols = 32;
+template <int ROWS>
 struct ColChunk {
-  v4f v[kColRows / 32];
+  static constexpr int kStride = ROWS + 4;
+  v4f v[ROWS / 32];
   __device__ static __forceinline__ int row(int k) {  // of thread 0..255's k-th group
     return 4 * (((threadIdx.x >> 5) & 7) + 8 * k);
   }
-  // rows [row0, row0 + 256) of column src (row stride ld); past the column's
+  // rows [row0, row0 + ROWS) of column src (row stride ld); past the column's
   // `rows` rows its last one
   __device__ __forceinline__ void fetch(const float* src, size_t ld, int row0, int rows) {
 #pragma unroll
-    for (int k = 0; k < kColRows / 32; k++)
+    for (int k = 0; k < ROWS / 32; k++)
 #pragma unroll
       for (int e = 0; e < 4; e++) v[k][e] = src[(size_t)min(row0 + row(k) + e, rows - 1) * ld];
     asm volatile("" ::: "memory");  // the loads are issued here, not where they are parked
   }
   // into LDS, zeros from row n of the chunk on
   __device__ __forceinline__ void stash(float* buf, int n) {
-    if (n < kColRows) {
+    if (n < ROWS) {
 #pragma unroll
-      for (int k = 0; k < kColRows / 32; k++)
+      for (int k = 0; k < ROWS / 32; k++)
 #pragma unroll
         for (int e = 0; e < 4; e++) v[k][e] = row(k) + e < n ? v[k][e] : 0.0f;
     }
 #pragma unroll
-    for (int k = 0; k < kColRows / 32; k++)
-      *reinterpret_cast<v4f*>(buf + (threadIdx.x & 31) * kColStride + row(k)) = v[k];
+    for (int k = 0; k < ROWS / 32; k++)
+      *reinterpret_cast<v4f*>(buf + (threadIdx.x & 31) * kStride + row(k)) = v[k];
   }
 };
 

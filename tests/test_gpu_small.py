@@ -197,11 +197,12 @@ def l2(v):
 
 @pytest.mark.parametrize("pooling", [0, 1, 2])
 @pytest.mark.parametrize("lens", [[1], [64, 63, 1], [65, 2], [512, 31, 300], [513, 1, 256, 257, 512],
-                                  [1030, 768, 33]])
+                                  [1030, 768, 33], [520] + [2] * 300])
 def test_pooling_in_row_order(gpu_ctx, lens, pooling):
     """Mean (float32, row after row), CLS and last-token pooling and the L2 scale
-    of the longest texts of each kernel and one more, bit for bit from the token
-    vectors of the same forward."""
+    of the longest texts of each kernel and one more, and of a long text whose
+    batch is too many for the chunked kernel, bit for bit from the token vectors
+    of the same forward."""
     say(f"pooling {pooling} lens={lens}")
     shape = BertShape("pool", layers=1, hidden=192, heads=6, intermediate=320, vocab=500,
                       max_position=1032, pooling=pooling, normalize=1)
@@ -216,12 +217,13 @@ def test_pooling_in_row_order(gpu_ctx, lens, pooling):
         assert np.array_equal(got[b], l2(v)), b
 
 
-@pytest.mark.parametrize("batch", [1, 3, 8, 9])
+@pytest.mark.parametrize("batch", [1, 3, 8, 9, 57, 90])
 @pytest.mark.parametrize("dense", [32, 300, 1056])
 def test_dense_head_in_order(gpu_ctx, batch, dense):
     """EmbeddingGemma's two head products, each output one float32 sum in
     ascending order, bit for bit from the token vectors; widths that leave
-    ragged chunks and column tiles, batches around a workgroup's 8 texts."""
+    ragged chunks and column tiles, batches around a workgroup's 8 texts and
+    past one round of the chip (for the first product, for both)."""
     say(f"dense head batch={batch} dense={dense}")
     shape = dataclasses.replace(GEMMA3_300M, name="head", layers=1, sliding_pattern=1, vocab=500,
                                 dense_hidden=dense)
