@@ -571,6 +571,7 @@ hipError_t launch_embed_layernorm(const EmbedArgs& a, int total, hipStream_t s) 
   else if (vec && v <= 2) hipLaunchKernelGGL((embed_ln_vec_kernel<2>), grid, block, 0, s, a, total);
   else if (vec && v <= 3) hipLaunchKernelGGL((embed_ln_vec_kernel<3>), grid, block, 0, s, a, total);
   else if (vec && v <= 4) hipLaunchKernelGGL((embed_ln_vec_kernel<4>), grid, block, 0, s, a, total);
+  else if (vec) hipLaunchKernelGGL((embed_ln_vec_kernel<8>), grid, block, 0, s, a, total);
   else hipLaunchKernelGGL(embed_ln_kernel, dim3(ceil_div(total, kRowsPerBlock)), dim3(256), 0, s,
                           a, total);
   return hipGetLastError();

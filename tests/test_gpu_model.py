@@ -69,6 +69,24 @@ def test_minilm_fp32_max_abs_1e4(gpu_ctx, minilm):
     assert err <= 1e-4
 
 
+@pytest.mark.parametrize("hidden", [1088, 2048])
+def test_hidden_wider_than_1024(gpu_ctx, hidden):
+    """The embedding LayerNorm writes the first projection's bf16 planes at
+    every width it takes: a fresh handle's first call against the oracle, and
+    the same call again after the buffers held another batch."""
+    from rembed_amd.synthetic import BertShape, bert_tensors, token_batch
+    shape = BertShape("wide", layers=1, hidden=hidden, heads=hidden // 64, intermediate=128,
+                      vocab=200, max_position=64)
+    t = bert_tensors(shape, seed=4)
+    ids, lens = token_batch(3, 40, 5, 40, vocab=200, id_lo=4, seed=6)
+    say(f"hidden {hidden}")
+    m, got = gpu_embed(gpu_ctx, shape, t, 0, ids, lens)
+    want = O.BertOracle(shape, t, 0).embed_batch(ids, lens, threads=8)
+    assert np.abs(got - want).max() <= 1e-4
+    m.embed(ids[::-1].copy(), lens[::-1].copy())
+    assert np.array_equal(m.embed(ids, lens), got)
+
+
 def test_minilm_weight_only_cosine(gpu_ctx, minilm):
     shape, t, ids, lens = minilm
     say("minilm w8")
