@@ -791,9 +791,10 @@ hipError_t launch_l2_rows(float* y, int rows, int H, hipStream_t s) {
   return hipGetLastError();
 }
 
-// Pooling and L2Normalize of one text per workgroup (H <= 2048: two columns per
-// thread), for short texts and CLS / last-token pooling: the arithmetic of
-// pool_kernel and l2_rows_kernel without the launch between them.
+// Pooling and L2Normalize of one text per workgroup (H <= 2048: one or two columns
+// per thread and no idle waves, see launch_pool), for short texts and CLS /
+// last-token pooling: the arithmetic of pool_kernel and l2_rows_kernel without the
+// launch between them.
 __global__ __launch_bounds__(1024) void pool_l2_kernel(const float* __restrict__ x, int H,
                                                        const int32_t* __restrict__ cu, int pooling,
                                                        float* __restrict__ out) {
@@ -804,7 +805,7 @@ __global__ __launch_bounds__(1024) void pool_l2_kernel(const float* __restrict__
   double part = 0.0;
 #pragma unroll
   for (int k = 0; k < 2; k++) {
-    const int j = threadIdx.x + 1024 * k;
+    const int j = threadIdx.x + blockDim.x * k;
     if (j >= H) continue;
     if (pooling == RH_POOL_MEAN) {
       const float* col = x + (size_t)r0 * H + j;
@@ -826,7 +827,7 @@ __global__ __launch_bounds__(1024) void pool_l2_kernel(const float* __restrict__
   const float inv = l2_scale(part, H, [&](int j) { return row[j]; });
 #pragma unroll
   for (int k = 0; k < 2; k++) {
-    const int j = threadIdx.x + 1024 * k;
+    const int j = threadIdx.x + blockDim.x * k;
     if (j < H) out[(size_t)b * H + j] = v[k] * inv;
   }
 }
@@ -863,7 +864,11 @@ hipError_t launch_pool(const float* x, int H, const int32_t* cu, const int32_t* 
   if (batch <= 0) return hipSuccess;
   const int kind = pick_pool(H, cu_host, batch, pooling, normalize);
   if (kind == POOL_L2) {
-    hipLaunchKernelGGL(pool_l2_kernel, dim3(batch), dim3(1024), 0, s, x, H, cu, pooling, out);
+    // as many waves as the columns take: with 1024 threads for 384 columns a CU held
+    // two texts (4096 texts of 1..8 rows 44 -> 20 µs, of 40..64 103 -> 85; with the
+    // two kernels 34 and 142)
+    const int threads = 64 * ceil_div(H > 1024 ? ceil_div(H, 2) : H, 64);
+    hipLaunchKernelGGL(pool_l2_kernel, dim3(batch), dim3(threads), 0, s, x, H, cu, pooling, out);
     return hipGetLastError();
   }
   if (kind == POOL_LONG)

@@ -217,6 +217,21 @@ def test_pooling_in_row_order(gpu_ctx, lens, pooling):
         assert np.array_equal(got[b], l2(v)), b
 
 
+@pytest.mark.parametrize("hidden", [64, 1024, 1088, 2048])
+def test_pooling_widths(gpu_ctx, hidden):
+    """One column per thread up to 1024 columns, two above, with the last wave
+    part empty: mean of short texts and the L2 scale, bit for bit."""
+    say(f"pooling hidden={hidden}")
+    shape = BertShape("wide", layers=1, hidden=hidden, heads=hidden // 64, intermediate=64,
+                      vocab=100, max_position=64, pooling=0, normalize=1)
+    m = Model(gpu_ctx, shape, bert_tensors(shape, seed=3), 0)
+    lens = np.array([5, 64, 1], np.int32)
+    ids = np.random.default_rng(hidden).integers(0, shape.vocab, (3, 64))
+    for v, t in zip(m.embed(ids, lens), m.embed_tokens(ids, lens)):
+        assert np.array_equal(v, l2(in_order(t, np.float32)
+                                    * (np.float32(1) / np.float32(len(t)))))
+
+
 @pytest.mark.parametrize("batch", [1, 3, 8, 9, 57, 90])
 @pytest.mark.parametrize("dense", [32, 300, 1056])
 def test_dense_head_in_order(gpu_ctx, batch, dense):
