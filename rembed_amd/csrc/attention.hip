@@ -327,18 +327,30 @@ __global__ __launch_bounds__(256, MINW) void attention_bf16_kernel(AttnArgs p) {
     v_chunk[j] = ((off % kRowB) >> 4) ^ (4 * attn_vswz<DH>(k_row[j]));
   }
   const size_t kvo = (size_t)p.k_off + kvh * DH, vvo = (size_t)p.v_off + kvh * DH;
-  // bf16 rows: DMA into the other buffer, waited for by the block's barrier
+  // bf16 rows: DMA into the other buffer, waited for by the block's barrier. All
+  // of K before V: row by row, planes of head dims 32 and 64 took 1-5 % longer
+  // (one text of 2048, 12 heads of 64: 58.1 µs against 54.8).
   auto issue = [&](int kb, int buf) {
 #pragma unroll
     for (int t = 0; t < T; t++) {
       uint8_t* sK = lds + buf * kStage + t * 2 * kKB;
-      const __bf16* base = t ? qkv_lo : qkv;
+      const __bf16* base = (t ? qkv_lo : qkv) + kvo;
 #pragma unroll
       for (int j = 0; j < kKLoads; j++) {
         const int kg = kb * KV + k_row[j];
-        const __bf16* row = base + (size_t)(r0 + (kg < len ? kg : len - 1)) * p.ldqkv;
-        lds_dma16(row + kvo + k_chunk[j] * 8, sK + (wave * kKLoads + j) * 1024);
-        lds_dma16(row + vvo + v_chunk[j] * 8, sK + kKB + (wave * kKLoads + j) * 1024);
+        lds_dma16(base + (size_t)(r0 + (kg < len ? kg : len - 1)) * p.ldqkv + k_chunk[j] * 8,
+                  sK + (wave * kKLoads + j) * 1024);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < T; t++) {
+      uint8_t* sV = lds + buf * kStage + t * 2 * kKB + kKB;
+      const __bf16* base = (t ? qkv_lo : qkv) + vvo;
+#pragma unroll
+      for (int j = 0; j < kKLoads; j++) {
+        const int kg = kb * KV + k_row[j];
+        lds_dma16(base + (size_t)(r0 + (kg < len ? kg : len - 1)) * p.ldqkv + v_chunk[j] * 8,
+                  sV + (wave * kKLoads + j) * 1024);
       }
     }
   };
@@ -752,8 +764,10 @@ __global__ __launch_bounds__(64 * kH256Waves) void attention_h256_kernel(AttnArg
 // with them the bits that its quantizers see).
 template <int DH, bool F32>
 constexpr int kKV3 = DH >= (F32 ? 64 : 128) ? 32 : kAttnKV;
-template <int DH>
-constexpr int kMinW3 = DH == 256 ? 1 : 2;
+// A cap of two waves only where registers need it: head dim 128, and fp32 rows
+// up to it; planes of head dims 32 and 64 fit without and are 1 % ahead uncapped.
+template <int DH, bool F32>
+constexpr int kMinW3 = DH == 128 || (F32 && DH < 128) ? 2 : 1;
 
 template <int DH>
 static hipError_t launch_attn_dh(const AttnArgs& a, int precision, hipStream_t s) {
@@ -761,8 +775,8 @@ static hipError_t launch_attn_dh(const AttnArgs& a, int precision, hipStream_t s
   const dim3 grid(8 * ceil_div(a.max_len, kAttnQ) * (a.heads / a.kv_heads) * ceil_div(units, 8));
   if (a.in_bf16 == 2) {  // hi/lo planes: the three-term products
     if (precision != 3 || !a.qkv_lo) return hipErrorInvalidValue;
-    timed_launch((attention_bf16_kernel<DH, 2, kKV3<DH, false>, false, kMinW3<DH>>), grid, dim3(256),
-                 0, s, a);
+    timed_launch((attention_bf16_kernel<DH, 2, kKV3<DH, false>, false, kMinW3<DH, false>>), grid,
+                 dim3(256), 0, s, a);
   } else if (a.in_bf16) {  // bf16 input carries no low half: one-term products
     // head dim 256: the 16x16x32 kernel (two waves per SIMD; 324 against 372
     // µs at EmbeddingGemma's global layer, 186 against 219 at its window-512
@@ -773,8 +787,8 @@ static hipError_t launch_attn_dh(const AttnArgs& a, int precision, hipStream_t s
       timed_launch((attention_bf16_kernel<DH, 1, kAttnKV, false, 1>), grid, dim3(256), 0, s, a);
   }
   else if (precision == 3)
-    timed_launch((attention_bf16_kernel<DH, 2, kKV3<DH, true>, true, kMinW3<DH>>), grid, dim3(256),
-                 0, s, a);
+    timed_launch((attention_bf16_kernel<DH, 2, kKV3<DH, true>, true, kMinW3<DH, true>>), grid,
+                 dim3(256), 0, s, a);
   else
     timed_launch((attention_bf16_kernel<DH, 1, kAttnKV, true, 1>), grid, dim3(256), 0, s, a);
   return hipGetLastError();
