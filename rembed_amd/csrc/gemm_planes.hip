@@ -55,8 +55,7 @@ __device__ __forceinline__ void wait_stages(int later) {
 // rows to p.qk_out; see GemmPlArgs).
 template <int BM, int BN, int NS, int AT, int BT, bool GLU, int BK, int WGM, int WGN, int LW = 0,
           bool QKN = false>
-__global__ __launch_bounds__(64 * (WGM * WGN + LW),
-                             QKN ? 4 : 1) void gemm_planes_kernel(GemmPlArgs p) {
+__global__ __launch_bounds__(64 * (WGM * WGN + LW)) void gemm_planes_kernel(GemmPlArgs p) {
   constexpr int NW = WGM * WGN;        // waves that multiply
   constexpr int NT = 64 * (NW + LW);   // threads
   constexpr int CPR = BK / 8;    // 16-byte chunks per row
@@ -264,47 +263,53 @@ __global__ __launch_bounds__(64 * (WGM * WGN + LW),
       const float* src0 = reinterpret_cast<const float*>(lds) +
                           (wm * WGN + c / WN) * 32 * kEpiStride + c % WN;
       typedef __bf16 v4bf __attribute__((ext_vector_type(4)));
-      // This wave's rows of the band: their cos/sin pieces are loaded before
-      // the first row's store, so no table load queues behind a store
-      // (vmcnt counts both in order).
-      constexpr int RPW = 32 / WGN;
-      v4f ccs[RPW], sns[RPW];
+      // This wave's rows of the band, RPW at a time: their cos/sin pieces are loaded
+      // before the first row's store, so no table load queues behind a store
+      // (vmcnt counts both in order). All eight at once would take 64 registers
+      // beside the accumulators not yet parked: 138 in all and one workgroup per
+      // CU, or spills at the 128 that two allow. With four it is 112.
+      constexpr int RPW = 4;
+      static_assert(32 / WGN % RPW == 0, "rows per wave and band");
 #pragma unroll
-      for (int k = 0; k < RPW; k++) {
-        const int wr = i * 32 + wn + k * WGN;  // row within the wave row (uniform)
-        const int pos = __builtin_amdgcn_readlane(qk_pos0, wr);
-        ccs[k] = *reinterpret_cast<const v4f*>(p.qk_cos + (size_t)pos * half + dp);
-        sns[k] = *reinterpret_cast<const v4f*>(p.qk_sin + (size_t)pos * half + dp);
-      }
+      for (int k0 = 0; k0 < 32 / WGN; k0 += RPW) {
+        v4f ccs[RPW], sns[RPW];
 #pragma unroll
-      for (int k = 0; k < RPW; k++) {
-        const int rr = wn + k * WGN;
-        v4f x = *reinterpret_cast<const v4f*>(src0 + rr * kEpiStride);
-        const int grow = grow_base + rr;
-        const bool ok = grow < p.M;
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          if (p.col_scales) x[e] = x[e] * qk_cs[e];
-          if (p.bias) x[e] = x[e] + qk_bs[e];
+        for (int k = 0; k < RPW; k++) {
+          const int wr = i * 32 + wn + (k0 + k) * WGN;  // row within the wave row (uniform)
+          const int pos = __builtin_amdgcn_readlane(qk_pos0, wr);
+          ccs[k] = *reinterpret_cast<const v4f*>(p.qk_cos + (size_t)pos * half + dp);
+          sns[k] = *reinterpret_cast<const v4f*>(p.qk_sin + (size_t)pos * half + dp);
         }
-        float ss = (x[0] * x[0] + x[1] * x[1]) + (x[2] * x[2] + x[3] * x[3]);
-        for (int o = lph >> 1; o >= 1; o >>= 1) ss += __shfl_xor(ss, o, 64);
-        v4bf* out = reinterpret_cast<v4bf*>(p.qk_out + (size_t)grow * p.ldc + gcol);
-        const v4f cc = ccs[k], sn = sns[k];
-        const float inv = rms_inv(ss, dh, p.qk_eps);
-        v4f xn, pn;
 #pragma unroll
-        for (int e = 0; e < 4; e++) xn[e] = x[e] * inv * qk_g[e];
+        for (int k = 0; k < RPW; k++) {
+          const int rr = wn + (k0 + k) * WGN;
+          v4f x = *reinterpret_cast<const v4f*>(src0 + rr * kEpiStride);
+          const int grow = grow_base + rr;
+          const bool ok = grow < p.M;
 #pragma unroll
-        for (int e = 0; e < 4; e++) pn[e] = __shfl_xor(xn[e], lph >> 1, 64);
-        v4f o;
+          for (int e = 0; e < 4; e++) {
+            if (p.col_scales) x[e] = x[e] * qk_cs[e];
+            if (p.bias) x[e] = x[e] + qk_bs[e];
+          }
+          float ss = (x[0] * x[0] + x[1] * x[1]) + (x[2] * x[2] + x[3] * x[3]);
+          for (int o = lph >> 1; o >= 1; o >>= 1) ss += __shfl_xor(ss, o, 64);
+          v4bf* out = reinterpret_cast<v4bf*>(p.qk_out + (size_t)grow * p.ldc + gcol);
+          const v4f cc = ccs[k], sn = sns[k];
+          const float inv = rms_inv(ss, dh, p.qk_eps);
+          v4f xn, pn;
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const float a = first ? xn[e] : pn[e], b = first ? pn[e] : xn[e];
-          o[e] = first ? a * cc[e] - b * sn[e] : b * cc[e] + a * sn[e];
+          for (int e = 0; e < 4; e++) xn[e] = x[e] * inv * qk_g[e];
+#pragma unroll
+          for (int e = 0; e < 4; e++) pn[e] = __shfl_xor(xn[e], lph >> 1, 64);
+          v4f o;
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const float a = first ? xn[e] : pn[e], b = first ? pn[e] : xn[e];
+            o[e] = first ? a * cc[e] - b * sn[e] : b * cc[e] + a * sn[e];
+          }
+          if (vh) o = x;
+          if (ok) *out = v4bf{(__bf16)o[0], (__bf16)o[1], (__bf16)o[2], (__bf16)o[3]};
         }
-        if (vh) o = x;
-        if (ok) *out = v4bf{(__bf16)o[0], (__bf16)o[1], (__bf16)o[2], (__bf16)o[3]};
       }
       __syncthreads();  // the next band overwrites the parked columns
     } else if constexpr (GLU) {
@@ -505,6 +510,9 @@ hipError_t launch_gemm_planes_qk(const GemmPlArgs& a, hipStream_t s) {
   if (a.N % 256 != 0 || a.lda % 64 != 0 || a.ldb % 64 != 0 || a.ldc % 4 != 0 || !a.qk_out ||
       !(a.qk_dh == 64 || a.qk_dh == 128 || a.qk_dh == 256) || is_glu(a.act))
     return hipErrorInvalidValue;
+  // µs on 256x256 tiles, here with eight rows of cos/sin at once, here (one stream):
+  // K = 768, N = 1280: M = 32768 155, 132, 125, M = 16384 100, 82, 74; K = 1024,
+  // N = 4096: M = 16384 222, 208, 198, M = 8192 110, 108, 104
   const int tiles = ceil_div(a.M, 128) * (a.N / 256);
   timed_launch((gemm_planes_kernel<128, 256, 3, 1, 1, false, 32, 2, 4, 0, true>), dim3(tiles),
                dim3(512), 0, s, a);

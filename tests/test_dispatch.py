@@ -1,9 +1,11 @@
-"""The host-side rules that choose a kernel, asked without a GPU.
+"""The host-side rules that choose a kernel, asked without a GPU, and the
+registers that the built kernels got.
 
 Each table row is a size at which the kernels were timed on MI355X, with the
 choices that came within 3 % of the fastest there (or within 0.3 us of it).
 """
 import ctypes
+import struct
 
 import pytest
 
@@ -58,3 +60,58 @@ def test_mean_pooling_kernel(h, lens, kernel):
     assert pick(h, cu, len(lens), 0, 0) == (LONG if kernel == LONG else ROWS)
     assert pick(h, cu, len(lens), 1, 1) == L2
     assert pick(h, cu, len(lens), 1, 0) == ROWS
+
+
+def built_kernels():
+    """The amdhsa metadata of every gfx950 kernel in the built library."""
+    import msgpack
+    from rembed_amd import _lib
+    blob, out, at = open(_lib.LIB_PATH, "rb").read(), {}, 0
+    while (at := blob.find(b"__CLANG_OFFLOAD_BUNDLE__", at)) >= 0:
+        p = at + 32
+        for _ in range(struct.unpack_from("<Q", blob, at + 24)[0]):
+            off, size, n = struct.unpack_from("<QQQ", blob, p)
+            target, p = blob[p + 24:p + 24 + n], p + 24 + n
+            if b"gfx950" not in target:
+                continue
+            elf = blob[at + off:at + off + size]
+            headers, = struct.unpack_from("<Q", elf, 32)
+            each, count = struct.unpack_from("<HH", elf, 54)
+            for h in range(headers, headers + each * count, each):
+                kind, _, q, _, _, length, _, _ = struct.unpack_from("<IIQQQQQQ", elf, h)
+                end = q + length
+                while kind == 4 and q < end:  # PT_NOTE
+                    nl, dl, note = struct.unpack_from("<III", elf, q)
+                    d = q + 12 + (nl + 3) // 4 * 4
+                    if note == 32:  # NT_AMDGPU_METADATA
+                        for k in msgpack.unpackb(elf[d:d + dl])["amdhsa.kernels"]:
+                            out[k[".name"]] = k
+                    q = d + (dl + 3) // 4 * 4
+        at += 24
+    return out
+
+
+# kernels that spill by design of their tile: the in-loop split, the GEMM that
+# finishes LayerNorm rows and the 256x256 int8 tiles on four or eight waves
+SPILL = ("gemm_bf16_kernel", "gemm_i8_ln_kernel", "gemm_i8_kernelILi256ELi256E")
+
+
+def test_no_kernel_spills():
+    kernels = built_kernels()
+    assert len(kernels) > 100
+    bad = [n for n, k in kernels.items()
+           if k[".private_segment_fixed_size"] and not any(s in n for s in SPILL)]
+    assert not bad, bad
+
+
+def test_planes_tiles_of_two_workgroups_fit_twice():
+    """512-thread planes kernels whose LDS fits a CU twice: at most 128 of a
+    SIMD lane's 512 registers, two workgroups being four waves on each."""
+    seen = 0
+    for n, k in built_kernels().items():
+        if "gemm_planes_kernel" not in n or k[".max_flat_workgroup_size"] != 512:
+            continue
+        if k[".group_segment_fixed_size"] <= 80 * 1024:
+            seen += 1
+            assert k[".vgpr_count"] <= 128, (n, k[".vgpr_count"])
+    assert seen > 10
