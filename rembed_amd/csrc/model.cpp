@@ -23,6 +23,13 @@
 
 using namespace rh;
 
+namespace rh {
+size_t staging_capacity(size_t have, size_t need, size_t most) {
+  const size_t grown = std::max<size_t>({need, std::min(2 * have, most), 1});
+  return round_up(grown, 1 << 16);
+}
+}  // namespace rh
+
 namespace {
 
 struct HostTensor {
@@ -462,10 +469,10 @@ struct rh_model {
   // The pinned landing place of `bytes` vectors and the events of its parts.
   int ensure_out_staging(size_t bytes, int parts) {
     if (!out_pinned || bytes > out_pinned_cap) {
+      const size_t cap = staging_capacity(out_pinned_cap, bytes, kOutStaged);
       if (out_pinned) RH_HIP(hipHostFree(out_pinned));
       out_pinned = nullptr;
       out_pinned_cap = 0;
-      const size_t cap = round_up(std::max<size_t>(bytes, 1), 1 << 16);
       RH_HIP(hipHostMalloc((void**)&out_pinned, 16 + cap));
       out_pinned_cap = cap;
     }

@@ -62,6 +62,21 @@ def test_mean_pooling_kernel(h, lens, kernel):
     assert pick(h, cu, len(lens), 1, 0) == ROWS
 
 
+def test_output_staging_grows_by_doubling():
+    """Outputs that grow by 64 KiB a call up to the 8 MiB that are staged pin
+    memory eight times, not at every call, and never more than they may."""
+    grow = rule("_ZN2rh16staging_capacityEmmm", *[ctypes.c_size_t] * 3)
+    grow.restype = ctypes.c_size_t
+    most, cap, pinned = 8 << 20, 0, 0
+    for need in range(1 << 16, most + 1, 1 << 16):
+        if need > cap:
+            cap, pinned = grow(cap, need, most), pinned + 1
+        assert need <= cap <= most
+    assert pinned == 8
+    assert grow(0, 0, most) == grow(0, 1, most) == 1 << 16
+    assert grow(0, most, most) == most and grow(5 << 20, 6 << 20, most) == most
+
+
 def built_kernels():
     """The amdhsa metadata of every gfx950 kernel in the built library."""
     import msgpack
