@@ -415,7 +415,9 @@ int rh_model_quantized_activations(const rh_model *m);
  * host int64 as the reference's Forward takes them (bert.go:649), text b is
  * ids[b*stride .. b*stride+lens[b]); out is [batch][H] host. An id outside
  * [0, vocab) returns RH_ERR_VOCAB (bert.go:797-800); batch*stride must be
- * below 2^31. Synchronous: the call returns with out filled. */
+ * below 2^31. Synchronous: the call returns with out filled; an error found
+ * before the forward runs leaves out as it was, after one of RH_ERR_HIP its
+ * contents are unspecified. */
 int rh_model_embed(rh_model *m, const int64_t *ids, const int32_t *lens,
                    int batch, int stride, float *out);
 /* EmbedTokens / ForwardTokens (rembed.go:370-411, bert.go:705-731): out is

@@ -140,4 +140,7 @@ int run_gemm_i8_ln(Context* ctx, const rh_weight* w, const uint8_t* qa, int ldq,
 // outputs grow a little at a time do not each pin memory anew (59 calls of 8 texts,
 // 40..504 tokens: 116 ms by exact sizes, 27 now).
 size_t staging_capacity(size_t have, size_t need, size_t most);
+// Faults in the pages of a host buffer for writing and leaves its bytes as they
+// are (also where another thread reads or writes them).
+void prefault(void* p, size_t bytes);
 }  // namespace rh

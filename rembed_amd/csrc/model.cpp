@@ -28,6 +28,18 @@ size_t staging_capacity(size_t have, size_t need, size_t most) {
   const size_t grown = std::max<size_t>({need, std::min(2 * have, most), 1});
   return round_up(grown, 1 << 16);
 }
+
+void prefault(void* p, size_t bytes) {
+  // a compare-exchange of 0 by 0 faults like a write and changes nothing; one in
+  // each page, the last one's too
+  auto touch = [](unsigned char* at) {
+    unsigned char zero = 0;
+    __atomic_compare_exchange_n(at, &zero, 0, false, __ATOMIC_RELAXED, __ATOMIC_RELAXED);
+  };
+  unsigned char* b = static_cast<unsigned char*>(p);
+  for (size_t i = 0; i < bytes; i += 4096) touch(b + i);
+  if (bytes) touch(b + bytes - 1);
+}
 }  // namespace rh
 
 namespace {
@@ -1998,10 +2010,9 @@ static int embed_common(rh_model* m, const int64_t* ids, const int32_t* lens, in
     if (e == hipSuccess && parts > 1) e = hipEventRecord(m->ev_out[p], s);
     at = end;
   }
-  // Touch the caller's pages while the forward runs: a fresh buffer's page faults
-  // would otherwise stand in the copies.
-  if (bytes >= 1 << 16)
-    for (size_t i = 0; i < bytes; i += 4096) reinterpret_cast<volatile char*>(out)[i] = 0;
+  // The caller's pages while the forward runs: a fresh buffer's page faults would
+  // otherwise stand in the copies.
+  if (e == hipSuccess && bytes >= 1 << 16) prefault(out, bytes);
   if (e == hipSuccess && !staged) e = hipMemcpyAsync(out, vec, bytes, hipMemcpyDeviceToHost, s);
   at = 0;
   for (int p = 0; p + 1 < parts && e == hipSuccess; p++) {

@@ -77,6 +77,18 @@ def test_output_staging_grows_by_doubling():
     assert grow(0, most, most) == most and grow(5 << 20, 6 << 20, most) == most
 
 
+@pytest.mark.parametrize("bytes_", [0, 1, 4095, 4096, 4097, 1 << 20])
+def test_prefault_leaves_the_buffer_as_it_was(bytes_):
+    """Pages are faulted in before the results exist: a call that then fails must
+    not have changed a reused buffer, nor anything beside it."""
+    touch = rule("_ZN2rh8prefaultEPvm", ctypes.c_void_p, ctypes.c_size_t)
+    touch.restype = None
+    was = bytes(i * 37 % 256 for i in range(4096)) * (bytes_ // 4096 + 2)
+    buf = ctypes.create_string_buffer(was, len(was))
+    touch(ctypes.addressof(buf) + 64, bytes_)
+    assert buf.raw == was
+
+
 def built_kernels():
     """The amdhsa metadata of every gfx950 kernel in the built library."""
     import msgpack
