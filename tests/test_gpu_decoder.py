@@ -53,16 +53,20 @@ def oracle_dense(mode, bT, a):
 # bf: the weight-only int8 / fp32 GEMM on pre-split bf16 planes (0) or with
 # the split in its main loop (1); full int8 has one path
 @pytest.mark.parametrize("mode,bf,tile", [(_lib.RH_MODE_F32, 0, 0), (_lib.RH_MODE_F32, 1, 0),
-                                          (_lib.RH_MODE_W8, 0, 0), (_lib.RH_MODE_W8, 1, 0),
-                                          (_lib.RH_MODE_W8, 0, 6), (_lib.RH_MODE_W8, 0, 10),
-                                          (_lib.RH_MODE_A8W8, 0, 0)],
-                         ids=["f32", "f32-inloop", "w8", "w8-inloop", "w8-tile6", "w8-tile10",
+                                          (_lib.RH_MODE_F32, 0, 1), (_lib.RH_MODE_F32, 0, 2),
+                                          (_lib.RH_MODE_F32, 0, 3), (_lib.RH_MODE_W8, 0, 0),
+                                          (_lib.RH_MODE_W8, 1, 0), (_lib.RH_MODE_W8, 0, 3),
+                                          (_lib.RH_MODE_W8, 0, 6), (_lib.RH_MODE_W8, 0, 8),
+                                          (_lib.RH_MODE_W8, 0, 10), (_lib.RH_MODE_A8W8, 0, 0)],
+                         ids=["f32", "f32-inloop", "f32-tile1", "f32-tile2", "f32-tile3", "w8",
+                              "w8-inloop", "w8-tile3", "w8-tile6", "w8-tile8", "w8-tile10",
                               "a8w8"])
 @pytest.mark.parametrize("act", [_lib.RH_ACT_SWIGLU, _lib.RH_ACT_GEGLU, _lib.RH_ACT_GEGLU_ERF],
                          ids=["swiglu", "geglu-tanh", "geglu-erf"])
 def test_gated_linear_matches_oracle(gpu_ctx, mode, bf, tile, act):
-    """Gated linear against the oracle; tile forces a planes tile (6 and 10
-    are the two the automatic choice gives large one-term GLU linears)."""
+    """Gated linear against the oracle; tile forces a planes tile that the
+    automatic choice gives larger GLU linears (one-term: 3, 6 = 1, 8 and 10;
+    fp32: 1, 2 and 3)."""
     ctx = gpu_ctx
     rng = np.random.default_rng(10 * mode + act)
     m, k, i = 301, 384, 528

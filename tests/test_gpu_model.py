@@ -12,6 +12,7 @@ import numpy as np
 import pytest
 
 from oracle import oracle as O
+from rembed_amd import _lib
 
 pytestmark = pytest.mark.gpu
 
@@ -150,7 +151,8 @@ def test_onepass_ffn1_identical(gpu_ctx, request, model, streams):
     for bit, as fp32 rows followed by the separate GELU + quantize pass.
     Repeated calls and a smaller batch after the full one check that every
     launch leaves its departure counts zero and its row slots empty for the
-    next; no wait timed out (rh_model_check)."""
+    next; no wait timed out (rh_model_check). The smaller batch also runs with
+    an int8 tile forced, which keeps calls of few rows on the one pass too."""
     from rembed_amd.model import Model
     shape, t, ids, lens = request.getfixturevalue(model)
     say(f"{shape.name}: {len(lens)} texts, {int(lens.sum())} rows, {streams} stream(s)")
@@ -163,6 +165,19 @@ def test_onepass_ffn1_identical(gpu_ctx, request, model, streams):
     for rep in range(3):
         assert np.array_equal(m.embed(ids, lens), plain), rep
         assert np.array_equal(m.embed(ids[:5], lens[:5]), few), rep
+    m.check()
+    gpu_ctx.set_option(_lib.RH_CTX_I8_TILE, 7)
+    try:
+        for rep in range(3):
+            for n, want in ((len(lens), plain), (5, few)):
+                gpu_ctx.profile(True)
+                got = m.embed(ids[:n], lens[:n])
+                onepass = gpu_ctx.profile_read(5)["launches"]
+                gpu_ctx.profile(False)
+                assert onepass >= shape.layers
+                assert np.array_equal(got, want), (rep, n)
+    finally:
+        gpu_ctx.set_option(_lib.RH_CTX_I8_TILE, 0)
     m.check()
 
 
