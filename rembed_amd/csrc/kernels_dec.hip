@@ -213,23 +213,22 @@ hipError_t launch_rms_residual(const RmsArgs& a, hipStream_t s) {
 // norm weights are null: nomic and ModernBERT rotate the raw projections,
 // nomic.go:210-211, modernbert.go:256-257), then rotate-half RoPE at the
 // row's position (applyRoPE, modernbert.go:130-143: each product rounded to
-// float32 before the add). With `outh` the results
-// go to bf16 rows of the same layout instead (round to nearest even), and
-// the v heads are converted too: the operands of a bf16 attention. With
-// `outl` as well, outh and outl receive the bf16 hi/lo split of the results,
-// the operands of an fp32-grade attention.
+// float32 before the add). The results go to bf16 rows `outh` of the same layout
+// (round to nearest even), and the v heads are converted too: the operands of a
+// bf16 attention. With `outl`, outh and outl receive the bf16 hi/lo split of the
+// results, the operands of an fp32-grade attention.
 // A wave takes kQkItems consecutive items, loading all of them before it
 // reduces, so their memory latencies overlap.
 constexpr int kQkItems = 4;
 
 __global__ __launch_bounds__(256) void qk_norm_rope_kernel(
-    float* __restrict__ qkv, int ldqkv, int m, int nq, int nkv, int dh,
+    const float* __restrict__ qkv, int ldqkv, int m, int nq, int nkv, int dh,
     const float* __restrict__ q_g, const float* __restrict__ k_g, float eps,
     const float* __restrict__ cos_t, const float* __restrict__ sin_t,
     const int32_t* __restrict__ pos, __bf16* __restrict__ outh, __bf16* __restrict__ outl) {
   const int lane = threadIdx.x & 63;
   const int item0 = (blockIdx.x * kRows + (threadIdx.x >> 6)) * kQkItems;
-  const int nh = nq + nkv + (outh ? nkv : 0);
+  const int nh = nq + 2 * nkv;
   const int total = m * nh;
   const int half = dh >> 1;
   // lane holds pairs (d, d + half) for d = lane, lane + 64 (dh <= 256)
@@ -250,8 +249,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(
     const int item = item0 + it;
     if (item >= total) return;
     const int row = item / nh, h = item % nh;
-    float* v = qkv + (size_t)row * ldqkv + h * dh;
-    __bf16* o = outh ? outh + (size_t)row * ldqkv + h * dh : nullptr;
+    __bf16* o = outh + (size_t)row * ldqkv + h * dh;
     __bf16* ol = outl ? outl + (size_t)row * ldqkv + h * dh : nullptr;
     auto store = [&](int d, float x) {
       __bf16 hi, lo;
@@ -286,13 +284,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(
         const float b = g ? x2[it][e] * inv * g[d + half] : x2[it][e];
         const float cc = c[d], ssn = sn[d];
         const float t0 = a * cc, t1 = b * ssn, t2 = b * cc, t3 = a * ssn;
-        if (o) {
-          store(d, t0 - t1);
-          store(d + half, t2 + t3);
-        } else {
-          v[d] = t0 - t1;
-          v[d + half] = t2 + t3;
-        }
+        store(d, t0 - t1);
+        store(d + half, t2 + t3);
       }
     }
   }
@@ -306,7 +299,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(
 // (only the sum of squares is added in another order).
 template <int DH>
 __global__ __launch_bounds__(256) void qk_norm_rope_vec_kernel(
-    float* __restrict__ qkv, int ldqkv, int nq, int nkv, const float* __restrict__ q_g,
+    const float* __restrict__ qkv, int ldqkv, int nq, int nkv, const float* __restrict__ q_g,
     const float* __restrict__ k_g, float eps, const float* __restrict__ cos_t,
     const float* __restrict__ sin_t, const int32_t* __restrict__ pos,
     __bf16* __restrict__ outh, __bf16* __restrict__ outl) {
@@ -317,8 +310,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_vec_kernel(
   const int row = blockIdx.x;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int l = lane % LPH, d = l * 4;
-  const int nh = nq + nkv + (outh ? nkv : 0);
-  float* rowp = qkv + (size_t)row * ldqkv;
+  const int nh = nq + 2 * nkv;
+  const float* rowp = qkv + (size_t)row * ldqkv;
   const int p = pos[row];
   for (int base = 0; base < nh; base += IT * 4 * HPW) {
     v4f x[IT];
@@ -365,20 +358,17 @@ __global__ __launch_bounds__(256) void qk_norm_rope_vec_kernel(
         const float a = first ? xn[c] : pn[c], b = first ? pn[c] : xn[c];
         o[c] = first ? a * cc[c] - b * sn[c] : b * cc[c] + a * sn[c];
       }
-      if (outh)
-        store_planes4(outh, outl, off, o);
-      else
-        *reinterpret_cast<v4f*>(qkv + off) = o;
+      store_planes4(outh, outl, off, o);
     }
   }
 }
 
-hipError_t launch_qk_norm_rope(float* qkv, int ldqkv, int m, int nq, int nkv, int dh,
+hipError_t launch_qk_norm_rope(const float* qkv, int ldqkv, int m, int nq, int nkv, int dh,
                                const float* q_g, const float* k_g, float eps,
                                const float* cos_t, const float* sin_t,
                                const int32_t* pos, __bf16* outh, __bf16* outl, hipStream_t s) {
   if (m <= 0) return hipSuccess;
-  if (dh % 2 || dh > 256 || (outl && !outh)) return hipErrorInvalidValue;
+  if (dh % 2 || dh > 256 || !outh) return hipErrorInvalidValue;
   const bool vec = ldqkv % 4 == 0 && ((reinterpret_cast<uintptr_t>(qkv) & 15) == 0) &&
                    ((reinterpret_cast<uintptr_t>(outh) & 7) == 0) &&
                    ((reinterpret_cast<uintptr_t>(outl) & 7) == 0);
@@ -394,7 +384,7 @@ hipError_t launch_qk_norm_rope(float* qkv, int ldqkv, int m, int nq, int nkv, in
                          nq, nkv, q_g, k_g, eps, cos_t, sin_t, pos, outh, outl);
     return hipGetLastError();
   }
-  const int items = m * (nq + nkv + (outh ? nkv : 0));
+  const int items = m * (nq + 2 * nkv);
   hipLaunchKernelGGL(qk_norm_rope_kernel, dim3(ceil_div(items, kRows * kQkItems)), dim3(256), 0,
                      s, qkv, ldqkv, m, nq, nkv, dh, q_g, k_g, eps, cos_t, sin_t, pos, outh, outl);
   return hipGetLastError();
@@ -502,7 +492,6 @@ hipError_t launch_dense_head(const float* pooled, int batch, int H, int D, const
                              const float* w2T, int normalize, float* hid, float* out,
                              hipStream_t s) {
   if (batch <= 0) return hipSuccess;
-  if ((size_t)std::max(H, D) * sizeof(float) > 64 * 1024) return hipErrorInvalidValue;
   launch_dense(w1T, H, D, batch, pooled, hid, s);
   launch_dense(w2T, D, H, batch, hid, out, s);
   hipError_t e = hipGetLastError();

@@ -438,9 +438,10 @@ struct RmsArgs {
 };
 hipError_t launch_rms_residual(const RmsArgs& a, hipStream_t s);
 // QK-norm (RMSNorm over each head's dh values; none when q_g and k_g are
-// null) then rotate-half RoPE at the row's position, in place on fused q|k
-// rows (qwen3.go:484-516; nomic.go:210-211, modernbert.go:256-257).
-hipError_t launch_qk_norm_rope(float* qkv, int ldqkv, int m, int nq, int nkv, int dh,
+// null) then rotate-half RoPE at the row's position over fused q|k|v rows
+// (qwen3.go:484-516; nomic.go:210-211, modernbert.go:256-257), v converted: bf16
+// rows to outh, or their hi/lo split to outh and outl.
+hipError_t launch_qk_norm_rope(const float* qkv, int ldqkv, int m, int nq, int nkv, int dh,
                                const float* q_g, const float* k_g, float eps,
                                const float* cos_t, const float* sin_t,
                                const int32_t* pos, __bf16* outh, __bf16* outl, hipStream_t s);
