@@ -229,8 +229,11 @@ __device__ __forceinline__ void attn_store_rows(const AttnArgs& p, const v16f (&
 // What bounds it: the softmax's VALU work and the matrix cores in turn (a wave's
 // scores, softmax and P·V depend on each other), so it lives on waves per SIMD.
 // Three-term blocks therefore hold 32 keys at head dims 128 and up (and of fp32
-// rows at 64): two 64-KiB workgroups per CU at head dim 128, where 64 keys left
-// one. Measured on MI355X
+// rows at 64): two 66-KiB workgroups per CU at head dim 128, where 64 keys left
+// one. (A grid of one workgroup per CU at most gains nothing from that: one text
+// of 2048, 16/8 causal heads of 128, planes, 102 µs against 93 with 64 keys. The
+// blocks stay 32 there too, or a text's bits would depend on its batch.)
+// Measured on MI355X
 // (µs; before: fp32 rows staged between two barriers, V transposed by 2-byte
 // stores; planes with 64-key blocks):
 //   fp32 rows, 24 texts of 33..512, 16 heads of 64            100 -> 61
@@ -789,7 +792,8 @@ static hipError_t launch_attn_dh(const AttnArgs& a, int precision, hipStream_t s
   else if (precision == 3)
     timed_launch((attention_bf16_kernel<DH, 2, kKV3<DH, true>, true, kMinW3<DH, true>>), grid,
                  dim3(256), 0, s, a);
-  else
+  else  // one wave per SIMD at head dims 128 and 256: the next block's fp32 rows are
+        // in registers, 64 of them at 128, where two waves would have to spill 8
     timed_launch((attention_bf16_kernel<DH, 1, kAttnKV, true, 1>), grid, dim3(256), 0, s, a);
   return hipGetLastError();
 }

@@ -433,10 +433,11 @@ hipError_t launch_pl(const GemmSmallArgs& a, hipStream_t s) {
 // terms take 16x16 only: their chain of instructions, not the loads, is what
 // a workgroup waits for, and it grows with the tile (fp32, K = 768, N = 768, 64
 // rows: 6.9 with 16x16, 9.6 with 32x16; 96 rows, 288 tiles: 9.7 against 9.0
-// tiled). The tiled int8 kernels' smallest tile is 128x128, so there 64x32 and
-// 64x64 are worth their grids too (K = 3072, N = 768: 349 rows 12.8 against
-// 26.7, 1213 rows 17.4 against 27.5; K = 768, N = 768, 700 rows 8.2 against
-// 12.2; 2400 rows, 456 tiles, 14.3 against 13.2).
+// tiled). int8 is worth the grids of 64x32 and 64x64 too: the tiled kernel that
+// runs otherwise, 64x256, has a twelfth to a quarter of the workgroups (µs, here
+// against 64x256: K = 3072, N = 768: 349 rows 12.9 - 19.1, 1344 rows 17.5 - 19.8;
+// K = 768, N = 768: 700 rows 8.3 - 10.0, 1344 rows 9.3 - 10.6; N = 3072: 320 rows
+// 8.9 - 10.7; past 256 tiles, 1408 rows of K = 768, N = 768, it takes 10.6).
 int pick_small_tile(int M, int N, int terms) {
   static const int rt[] = {1, 2, 2, 4, 4}, ct[] = {1, 1, 2, 2, 4};
   const int most = terms == 0 ? 5 : terms == 2 ? 3 : 1;

@@ -885,12 +885,14 @@ int rh_model::forward_bert(const int32_t* ids_dev, int stride, const std::vector
                        L.f2->d_bias, nullptr, nullptr, 2.0 * MH * I * H);
       if (st) return st;
     } else if (qf1 && needs_q(L.f2)) {
-      // FFN1 writes the fp32 pre-activation (dequant + bias); GELU moves into
-      // FFN2's row quantizer, which has VALU to spare where the GEMM
-      // epilogue does not. Same float32 operations in the same order as
+      // The separate form: FFN1 writes the fp32 pre-activation (dequant + bias);
+      // GELU moves into FFN2's row quantizer, which has VALU to spare where the
+      // GEMM epilogue does not. Same float32 operations in the same order as
       // GELU(dense(x)) then QuantizeRowU8 (bert.go:910-916).
-      // few rows: FFN1 on the few-row kernel and the separate quantizer (28
-      // rows, 768x3072: 5.5 + 3.5 µs against 17.6 in one pass)
+      // few rows: FFN1 on the few-row kernel and the separate quantizer (28 rows,
+      // 768x3072: 5.5 + 3.5 µs against 17.6 in one pass), up to where that kernel
+      // ends: four BERT-base layers of 320 rows 230 µs against 268, four MiniLM
+      // layers of 640 201 against 236
       const bool few = ctx->i8_tile == 0 && pick_small_tile(Mp, I, 0) != 0;
       if (fused_ffn1 == 2 && I <= 256 * kQsyncMaxTiles && !few) {
         // one pass: FFN1's workgroups exchange the GELU rows' |max| per row
@@ -1749,7 +1751,10 @@ int rh_model_create(rh_context* ctx, const rh_model_config* cfg, int quant, rh_m
     m->quant = quant;
     // fp32-grade attention (the reference's attention is float32) for the
     // BERT family in every mode; the RoPE family's quantized modes keep bf16
-    // operands (their dh-256 fp32-grade kernel is the unpipelined one)
+    // operands: their one-term linears round every activation to bf16 anyway, and
+    // attention takes half to a third of the time (planes against bf16 rows: 24
+    // causal texts of 33..512, 16/8 heads of 128 78 and 42 µs; 6 texts of
+    // 300..2048, 3/1 heads of 256, fp32 rows 478 and 150)
     m->attn_precision = quant == RH_QUANT_NONE || bert_family ? 3 : 1;
     *out = m;
     return RH_OK;
