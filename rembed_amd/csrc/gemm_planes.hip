@@ -171,43 +171,81 @@ __global__ __launch_bounds__(64 * (WGM * WGN + LW)) void gemm_planes_kernel(Gemm
               f.a[x == BT ? 1 : 0][i], f.b[x == 1 && BT == 2 ? 1 : 0][j], acc[i][j], 0, 0, 0);
   };
 
+  // The one-term 256x256 tile keeps no fragments past a step: its 128 accumulators
+  // leave the compiler to place a stage's reads by itself, and holding the next
+  // step's across the barrier took 1-4 % longer (M = 16384: K = 768, N = 3072 104 µs
+  // against 100, K = 3072, N = 768 99 against 96). Its next stage is requested as a
+  // stage begins.
+  constexpr bool kPlain = AT + BT == 2 && BM == 256 && BN == 256;
+  if constexpr (kPlain) {
+    static_assert(NS == 2, "two stages");
+    issue(0);
+    for (int kt = 0; kt < nk; kt++) {
+      wait_vmcnt<0>();   // stage kt has landed for this wave,
+      wait_lgkmcnt0();   // which has read all of stage kt - 1,
+      stage_barrier();   // and so has and did every other
+      if (kt + 1 < nk) issue(kt + 1);
+      const uint8_t* sA = lds + (kt % NS) * kStage;
+      const uint8_t* sB = sA + kA;
 #pragma unroll
-  for (int st = 0; st < NS; st++)
-    if (st < nk) issue(st);
-  wait_stages<kLoads, NS - 1>(nk - 1);  // stage 0 has landed for this wave
-  stage_barrier();                      // and for the others
-  // To stage kt + 1: this wave's loads of it have landed once only those of the
-  // later stages issued are pending. Past the barrier that holds for every wave
-  // (a __syncthreads() fence would drain the ring) and all reads of stage kt are
-  // done, so its slot can be refilled.
-  auto advance = [&](int kt) {
-    wait_stages<kLoads, NS - 2>(nk - 2 - kt);
-    stage_barrier();
-    if (kt + NS < nk) issue(kt + NS);
-  };
-  if (LW > 0 && wave >= NW) {
-    for (int kt = 0; kt + 1 < nk; kt++) advance(kt);
-  } else {
-    constexpr int S = BK / 16;
-    Frags f[2];
-    read(f[0], 0, 0);
-    for (int kt = 0; kt + 1 < nk; kt++) {
+      for (int s = 0; s < BK / 16; s++) {
+        const int c = 2 * s + fg;
+        v8bf fa[TM], fb[TN];
 #pragma unroll
-      for (int s = 0; s < S; s++) {
-        if (s + 1 < S) {
-          read(f[(s + 1) & 1], kt, s + 1);
-        } else {
-          wait_lgkmcnt0();
-          advance(kt);
-          read(f[0], kt + 1, 0);
-        }
-        multiply(f[s & 1]);
+        for (int i = 0; i < TM; i++)
+          fa[i] = *reinterpret_cast<const v8bf*>(
+              sA + stage_frag_off<BK * 2>(wm * WM + i * 32 + fr, c));
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+          fb[j] = *reinterpret_cast<const v8bf*>(
+              sB + stage_frag_off<BK * 2>(wn * WN + j * 32 + fr, c));
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+          for (int j = 0; j < TN; j++)
+            acc[i][j] =
+                __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
       }
     }
+  } else {
 #pragma unroll
-    for (int s = 0; s < S; s++) {
-      if (s + 1 < S) read(f[(s + 1) & 1], nk - 1, s + 1);
-      multiply(f[s & 1]);
+    for (int st = 0; st < NS; st++)
+      if (st < nk) issue(st);
+    wait_stages<kLoads, NS - 1>(nk - 1);  // stage 0 has landed for this wave
+    stage_barrier();                      // and for the others
+    // To stage kt + 1: this wave's loads of it have landed once only those of the
+    // later stages issued are pending. Past the barrier that holds for every wave
+    // (a __syncthreads() fence would drain the ring) and all reads of stage kt are
+    // done, so its slot can be refilled.
+    auto advance = [&](int kt) {
+      wait_stages<kLoads, NS - 2>(nk - 2 - kt);
+      stage_barrier();
+      if (kt + NS < nk) issue(kt + NS);
+    };
+    if (LW > 0 && wave >= NW) {
+      for (int kt = 0; kt + 1 < nk; kt++) advance(kt);
+    } else {
+      constexpr int S = BK / 16;
+      Frags f[2];
+      read(f[0], 0, 0);
+      for (int kt = 0; kt + 1 < nk; kt++) {
+#pragma unroll
+        for (int s = 0; s < S; s++) {
+          if (s + 1 < S) {
+            read(f[(s + 1) & 1], kt, s + 1);
+          } else {
+            wait_lgkmcnt0();
+            advance(kt);
+            read(f[0], kt + 1, 0);
+          }
+          multiply(f[s & 1]);
+        }
+      }
+#pragma unroll
+      for (int s = 0; s < S; s++) {
+        if (s + 1 < S) read(f[(s + 1) & 1], nk - 1, s + 1);
+        multiply(f[s & 1]);
+      }
     }
   }
 
